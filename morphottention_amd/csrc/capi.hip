@@ -87,6 +87,16 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   d.B = (int)B;
   d.N = (int)N;
   d.NP = (int)((N + 63) / 64 * 64);
+  // The projection's rows of one batch row are padded to whole groups of 8
+  // tokens, so that its epilogue writes V^T and the remainders of 8 tokens of
+  // one column at a time, whatever N is: the padding rows repeat a token and
+  // their values are stored as the zeros that the V^T layout wants there. (With
+  // unpadded rows every value of a length that 8 does not divide was a 2-byte
+  // store: proj_fwd at B64 N197 D768 H12 m64 142 us, padded 79 us with the same
+  // epilogue.) From 32 tokens on the padding is at most a quarter of the rows;
+  // shorter rows keep their own rows and the element stores.
+  d.NR = (int)(N >= 32 ? (N + 7) / 8 * 8 : N);
+  d.TR = B * (int64_t)d.NR;
   d.D = (int)D;
   d.H = (int)H;
   d.M = (int)M;
@@ -106,14 +116,22 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   // of 160 or 128 columns (whichever divides H*M + D and needs fewer rounds
   // times tile area; 160 on a tie): e.g. H*M + D = 640, T = 8192 gives 256
   // workgroups of 128 x 160 (one round) instead of 320 of 128 x 128. The
-  // interleaved column order needs whole heads and 8-column pieces per tile.
+  // interleaved column order needs whole heads and 16-column blocks per tile,
+  // and a tile whose width is no multiple of m (160 at m = 64) needs that order,
+  // or heads would straddle tiles.
   const int NC = d.HM + d.D;
+  // tiles of bn columns (bn divides NC) can share the code and value columns
+  // evenly: whole heads and whole 16-column blocks each
+  auto whole_heads = [&](int bn) {
+    const int ntn = NC / bn;
+    return d.HM % ntn == 0 && d.D % ntn == 0 && (d.HM / ntn) % d.M == 0 && (d.D / ntn) % 16 == 0;
+  };
   d.PBN = NC % 320 == 0 ? 320 : 256;
-  if (((T + 255) / 256) * ((NC + d.PBN - 1) / d.PBN) < 256) {
-    const int64_t rows = (T + 127) / 128;
+  if (((d.TR + 255) / 256) * ((NC + d.PBN - 1) / d.PBN) < 256) {
+    const int64_t rows = (d.TR + 127) / 128;
     int64_t best = -1;
     for (const int bn : {160, 128}) {
-      if (NC % bn) continue;
+      if (NC % bn || (bn % d.M && !whole_heads(bn))) continue;
       const int64_t cost = (rows * (NC / bn) + 255) / 256 * bn;
       if (best < 0 || cost < best) {
         best = cost;
@@ -121,14 +139,15 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
       }
     }
   }
+  d.PGW = d.PBN;
   d.PCPT = d.PVPT = 0;
-  if (NC % d.PBN == 0) {
+  if (NC % d.PBN == 0 && whole_heads(d.PBN)) {
     const int ntn = NC / d.PBN;
-    if (d.HM % ntn == 0 && d.D % ntn == 0 && (d.HM / ntn) % d.M == 0 && (d.HM / ntn) % 8 == 0 &&
-        (d.D / ntn) % 8 == 0) {
-      d.PCPT = d.HM / ntn;
-      d.PVPT = d.D / ntn;
-    }
+    // half-tile groups where both halves are whole 16-column blocks
+    const int half = d.NR % 8 == 0 && (d.HM / ntn) % 32 == 0 && (d.D / ntn) % 32 == 0 ? 2 : 1;
+    d.PGW = d.PBN / half;
+    d.PCPT = d.HM / ntn / half;
+    d.PVPT = d.D / ntn / half;
   }
   return MORPHO_OK;
 }

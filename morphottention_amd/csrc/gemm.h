@@ -31,6 +31,8 @@
 // discarded outputs; k past kend is zeroed in LDS on the last k-step.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace morpho {
@@ -62,25 +64,29 @@ struct OpTile {
   }
 
   // Byte offset of the chunk from the tile's base (operand at row0, k0), with
-  // rows clamped into [0, rmax): rows past the extent re-read a valid row and
-  // only feed discarded outputs. Fits 32 bits for ld <= 65536.
-  __device__ __forceinline__ static unsigned lane_off(int64_t ld, int rmax, int piece, int lane) {
+  // rows clamped below nrows: rows past the extent re-read a valid row and
+  // only feed discarded outputs. Fits 32 bits for ld <= 65536. KC rows go
+  // through `map` (tile row space -> memory row).
+  template <class Map>
+  __device__ __forceinline__ static unsigned lane_off(int64_t ld, int row0, int nrows, int piece, int lane,
+                                                      const Map& map) {
     int r, k8;
     chunk(64 * piece + lane, r, k8);
-    if (KC) return (unsigned)(((int64_t)min(r, rmax - 1) * ld + k8) * 2);
-    return (unsigned)(((int64_t)k8 * ld + min(r, rmax - 8)) * 2);
+    if (KC) return (unsigned)(((int64_t)(map(min(row0 + r, nrows - 1)) - map(row0)) * ld + k8) * 2);
+    return (unsigned)(((int64_t)k8 * ld + min(r, nrows - row0 - 8)) * 2);
   }
   __device__ __forceinline__ static const char* tile_base(const f16* p, int64_t ld, int row0, int k0) {
     return reinterpret_cast<const char*>(KC ? p + (int64_t)row0 * ld + k0 : p + (int64_t)k0 * ld + row0);
   }
-  // Full address with k clamped into [k0, kend) as well (the ragged last
-  // k-step). KC needs kend % 8 == 0; KM needs nrows % 8 == 0.
-  __device__ __forceinline__ static const f16* tail_src(const f16* p, int64_t ld, int row0, int nrows, int k0,
-                                                        int kend, int piece, int lane) {
+  // Address of a chunk of the ragged last k-step (base: the operand at row0,
+  // k0; off: lane_off), with k clamped below kend as well. KC needs kend % 8
+  // == 0; KM needs nrows % 8 == 0.
+  __device__ __forceinline__ static const f16* tail_src(const char* base, unsigned off, int64_t ld, int k0, int kend,
+                                                        int piece, int lane) {
     int r, k8;
     chunk(64 * piece + lane, r, k8);
-    if (KC) return p + (int64_t)min(row0 + r, nrows - 1) * ld + min(k0 + k8, kend - 8);
-    return p + (int64_t)min(k0 + k8, kend - 1) * ld + min(row0 + r, nrows - 8);
+    const int over = KC ? max(0, k0 + k8 - (kend - 8)) : max(0, k0 + k8 - (kend - 1));  // k's to step back
+    return reinterpret_cast<const f16*>(base + off - 2 * (int64_t)over * (KC ? 1 : ld));
   }
 
   // Zero the k >= kvalid part of a stage tile (kvalid < BK; last k-step only).
@@ -110,6 +116,11 @@ struct OpTile {
       return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   }
+};
+
+// Row map of an operand whose tile rows are its memory rows.
+struct SameRows {
+  __device__ __forceinline__ int operator()(int r) const { return r; }
 };
 
 template <int BM, int BN, int WM, bool AKC, bool BKC, int BK = 32, int STAGES = 4>
@@ -148,9 +159,14 @@ struct Gemm {
   // tile; acc[i][j][r] holds C row m0 + WTM * (w / WN) + 16 i + 4 (lane / 16) + r,
   // column n0 + WTN * (w % WN) + 16 j + lane % 16.
   // Operands: A (M rows) and B (N rows = columns of C), each one matrix
-  // (p, ld); k runs over [kbeg, kend). lds: kLdsBytes, 16-byte aligned.
+  // (p, ld); k runs over [kbeg, kend). lds: kLdsBytes, 16-byte aligned. mapA
+  // (k-contiguous A only): the memory row of each of the M rows,
+  // nondecreasing, at most as far apart as the rows themselves.
+  template <class MapA = SameRows>
   __device__ __forceinline__ static void run(const f16* Ap, int64_t lda, const f16* Bp, int64_t ldb, int M, int N,
-                                             int m0, int n0, int kbeg, int kend, char* lds, f32x4 (&acc)[FI][FJ]) {
+                                             int m0, int n0, int kbeg, int kend, char* lds, f32x4 (&acc)[FI][FJ],
+                                             const MapA& mapA = MapA()) {
+    static_assert(AKC || std::is_same<MapA, SameRows>::value, "row maps are for k-contiguous operands");
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = w / WN, wn = w % WN;
 #pragma unroll
@@ -164,12 +180,12 @@ struct Gemm {
     // this wave's pieces: A pieces w + 8 i, B pieces w + 8 i (< TB::kDma)
     unsigned offA[kPA], offB[kPBmax];
 #pragma unroll
-    for (int i = 0; i < kPA; ++i) offA[i] = TA::lane_off(lda, M - m0, w + kGemmWaves * i, lane);
+    for (int i = 0; i < kPA; ++i) offA[i] = TA::lane_off(lda, m0, M, w + kGemmWaves * i, lane, mapA);
 #pragma unroll
     for (int i = 0; i < kPBmax; ++i)
-      offB[i] = TB::lane_off(ldb, N - n0, min(w + kGemmWaves * i, TB::kDma - 1), lane);
+      offB[i] = TB::lane_off(ldb, n0, N, min(w + kGemmWaves * i, TB::kDma - 1), lane, SameRows());
     const int64_t stepA = AKC ? 2 * kBK : 2 * kBK * lda, stepB = BKC ? 2 * kBK : 2 * kBK * ldb;  // bytes per k-step
-    const char* baseA = TA::tile_base(Ap, lda, m0, kbeg);
+    const char* baseA = TA::tile_base(Ap, lda, AKC ? mapA(m0) : m0, kbeg);
     const char* baseB = TB::tile_base(Bp, ldb, n0, kbeg);
 
     auto issue = [&](int t) {
@@ -187,12 +203,12 @@ struct Gemm {
       } else {
 #pragma unroll
         for (int i = 0; i < kPA; ++i)
-          lds_dma16(TA::tail_src(Ap, lda, m0, M, k0, kend, w + kGemmWaves * i, lane),
+          lds_dma16(TA::tail_src(baseA + t * stepA, offA[i], lda, k0, kend, w + kGemmWaves * i, lane),
                     st + 1024u * (unsigned)(w + kGemmWaves * i));
 #pragma unroll
         for (int i = 0; i < kPBmax; ++i)
           if (w + kGemmWaves * i < TB::kDma)
-            lds_dma16(TB::tail_src(Bp, ldb, n0, N, k0, kend, w + kGemmWaves * i, lane),
+            lds_dma16(TB::tail_src(baseB + t * stepB, offB[i], ldb, k0, kend, w + kGemmWaves * i, lane),
                       st + (unsigned)TA::kBytes + 1024u * (unsigned)(w + kGemmWaves * i));
       }
     };

@@ -16,6 +16,9 @@ struct Dims {
   int B, N, D, H, M, DV;  // batch, tokens, model dim, heads, cube_m, head_dim_v
   int NP;                 // N rounded up to a multiple of 64: row length of the V^T layout
   int64_t T;              // B * N tokens
+  int NR;                 // rows per batch row in the forward projection's row space: N, or N rounded up
+                          // to a multiple of 8 (make_dims)
+  int64_t TR;             // B * NR rows of that space
   int HM;                 // H * M projection columns
   int CW;                 // 2 * M + 8: code row width (hi/lo split codes + affine augmentation)
   float scale;
@@ -24,23 +27,19 @@ struct Dims {
   int proj;               // cube projection: kProjSigmoid, kProjHardTanh01 or kProjIdentity
   int det;                // deterministic backward: dq and row sums from per-key-block partials
   // Column order of the forward projection's B operand (wt rows): tiles of
-  // PBN columns; when PCPT > 0 tile j holds code columns [j PCPT, (j+1) PCPT)
-  // then value columns [j PVPT, (j+1) PVPT), so every tile does the same
+  // PBN columns in groups of PGW (whole or half tiles); when PCPT > 0 group g
+  // holds code columns [g PCPT, (g+1) PCPT) then value columns [g PVPT, (g+1)
+  // PVPT), so every tile (and, with half tiles, every wave) does the same
   // epilogue work; PCPT == 0 keeps the natural order [W_phi | W_V].
-  int PBN, PCPT, PVPT;
+  int PBN, PGW, PCPT, PVPT;
 };
 
-// Original [W_phi | W_V] column of local column lc of projection tile tn.
-__host__ __device__ inline int proj_col(const Dims& d, int tn, int lc) {
-  if (d.PCPT == 0) return tn * d.PBN + lc;
-  return lc < d.PCPT ? tn * d.PCPT + lc : d.HM + tn * d.PVPT + (lc - d.PCPT);
-}
-// wt row (position in the projection's column order) of original column c.
+// wt row (position in the projection's column order) of [W_phi | W_V] column c.
 __host__ __device__ inline int proj_row(const Dims& d, int c) {
   if (d.PCPT == 0) return c;
-  if (c < d.HM) return (c / d.PCPT) * d.PBN + c % d.PCPT;
+  if (c < d.HM) return (c / d.PCPT) * d.PGW + c % d.PCPT;
   const int v = c - d.HM;
-  return (v / d.PVPT) * d.PBN + d.PCPT + v % d.PVPT;
+  return (v / d.PVPT) * d.PGW + d.PCPT + v % d.PVPT;
 }
 
 // Products of the forward projection; the forward workspace holds exactly these.

@@ -72,12 +72,19 @@ hipError_t launch_transpose_weights(const Dims& d, const f16* W_phi, const f16* 
 // H*M + D columns (e.g. 1280 at B4 N4096 D1024 H16 m16, which makes the grid
 // exactly one round of 256 tiles), 256 x 256 otherwise, and 128 x 128 when
 // the large tiles would leave most CUs idle (few tokens: B8 N1024 D512 H8 m16
-// has 64 large tiles, 320 small ones). The epilogue takes the tile through
-// LDS in 64-row slabs (a slab holds the accumulators of the wave rows whose
-// rows it covers), fp32 with row stride BN + 5 = 5 (mod 64) banks: the value
-// pass below reads 8 rows x 8 columns per wave instruction on 64 distinct
-// banks, and the accumulator stores (16 columns x 4 row groups) are at most
-// 2-way.
+// has 64 large tiles, 320 small ones).
+//
+// Epilogue: the values leave straight from the accumulators (lane swaps
+// assemble 16-byte stores), the codes through LDS, and no wave waits for
+// another's values. What bounds it is the burst of its stores (B4 N4096 D1024
+// H16 m16: 97 MB at the end of one round of tiles) and, for code that runs
+// once per tile, instruction fetch: the value part is unrolled over a wave's
+// column blocks and loses 6 us there if each block carries its own slow paths.
+// Until now 64-row slabs of the whole tile went through LDS in fp32, two of the
+// eight waves writing at a time; proj_fwd in us, before -> after: B64 N197 D768
+// H12 m64 142 -> 80, B3 N1500 D1024 H8 m32 42.7 -> 23.8, B64 N128 D1024 H16 m16
+// 40.0 -> 31.0, B64 N1024 D768 H12 m64 256 -> 246, B4 N4096 D1024 H16 m16 55.4
+// -> 56.0 (the first two mostly from the padded rows, make_dims).
 template <int BM, int BN>
 using ProjGemm = Gemm<BM, BN, 4, true, true, 64, 2>;
 
@@ -92,20 +99,38 @@ using ProjGemm = Gemm<BM, BN, 4, true, true, 64, 2>;
 // (bit-identical, over every 7th float bit pattern of both signs, to the
 // nearest conversion stepped one code toward zero where that overshot).
 __device__ __forceinline__ float vlo_scaled(float r) { return fminf(fmaxf(r * (float)(1 << kVloExp), -448.f), 448.f); }
-__device__ __forceinline__ unsigned vlo_code(float r) {
-  return (unsigned)__builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r), 0, 0, 0) & 0xffu;
+// the codes of four remainders, byte k of the dword = r[k]
+__device__ __forceinline__ unsigned vlo_pack4(const float (&r)[4]) {
+  int w = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[0]), 0, 0, 0);
+  w = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[1]), 0, w, 1);
+  w = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[2]), 0, w, 2);
+  return (unsigned)__builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[3]), 0, w, 3);
 }
-__device__ __forceinline__ uint2 vlo_pack8(const float (&r)[8]) {
-  int w[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {  // byte k of the dword = r[4 i + k]
-    w[i] = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[4 * i]), 0, 0, 0);
-    w[i] = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[4 * i + 1]), 0, w[i], 1);
-    w[i] = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[4 * i + 2]), 0, w[i], 2);
-    w[i] = __builtin_amdgcn_cvt_sr_fp8_f32(vlo_scaled(r[4 * i + 3]), 0, w[i], 3);
+// v_permlane16_swap: the odd 16-lane rows of a change places with the even
+// ones of b (a' = a0 b0 a2 b2, b' = a1 b1 a3 b3).
+__device__ __forceinline__ void swap16(unsigned& a, unsigned& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// Lanes 8..15 of each 16-lane row of a change places with lanes 0..7 of b.
+__device__ __forceinline__ void swap8(unsigned& a, unsigned& b, bool upper) {
+  const unsigned send = upper ? a : b;
+  const unsigned got = (unsigned)__builtin_amdgcn_mov_dpp((int)send, 0x128 /* row_ror:8 */, 0xf, 0xf, false);
+  a = upper ? got : a;
+  b = upper ? b : got;
+}
+
+// Memory row (token) of a row of the projection's row space: batch rows of NR
+// rows, the last NR - N of which repeat the batch row's last token.
+struct TokenRows {
+  int NR, N;
+  __device__ __forceinline__ int operator()(int r) const {
+    const int b = r / NR;
+    return b * N + min(r - b * NR, N - 1);
   }
-  return make_uint2((unsigned)w[0], (unsigned)w[1]);
-}
+};
 
 // GEN: a cube projection other than the sigmoid, or the masked diagonal (the
 // variants take the projection from d.proj and the exact row maximum)
@@ -114,69 +139,174 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
                                                                const f16* __restrict__ gate_q,
                                                                const f16* __restrict__ gate_k, Dims d, ProjBuffers p) {
   using G = ProjGemm<BM, BN>;
-  constexpr int SS = BN + 5;  // stage row stride (floats)
-  // epilogue LDS: the 64-row slab, then the tile's gate products G = gq gk
-  static_assert(64 * SS * 4 + BN * 4 <= G::kLdsBytes, "epilogue slab and gate table must fit the main loop's LDS");
+  static_assert(64 * (BN + 4) * 4 + BN * 4 <= G::kLdsBytes, "a pass of 64 code rows and the gates must fit the LDS");
+  static_assert(G::WTM == 16 * G::FI && G::FI % 2 == 0 && G::WTM * 4 == BM, "four wave rows of whole block pairs");
   __shared__ __align__(16) char smem[G::kLdsBytes];
   constexpr int CW = 2 * M + 8;
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w / G::WN, wn = w % G::WN;
   const int NC = d.HM + d.D;
-  const int T = (int)d.T;
+  const int TR = (int)d.TR;
   int tm, tn;
-  if (!gemm_tile_map(blockIdx.x, (T + BM - 1) / BM, (NC + BN - 1) / BN, tm, tn)) return;
+  if (!gemm_tile_map(blockIdx.x, (TR + BM - 1) / BM, (NC + BN - 1) / BN, tm, tn)) return;
   const int n0 = tn * BN, m0 = tm * BM;
   f32x4 acc[G::FI][G::FJ];
-  G::run(X, d.D, p.wt, d.D, T, NC, m0, n0, 0, d.D, smem, acc);
+  G::run(X, d.D, p.wt, d.D, TR, NC, m0, n0, 0, d.D, smem, acc, TokenRows{d.NR, d.N});
 
-  float* stage = reinterpret_cast<float*>(smem);
-  float* gtab = stage + 64 * SS;
-  const float c1 = 2.0f * d.scale * kLog2e;
-  static_assert(G::WTM == 64 || G::WTM == 32, "wave rows of 64 or 32 rows");
-  // Code columns of this tile: local columns [0, ncode), whole heads (PCPT per
-  // tile in the interleaved order; in the natural order those below HM).
-  const int ncode = d.PCPT > 0 ? d.PCPT : max(0, min(BN, d.HM - n0));
-  // Gate products of the code columns, read from global memory once per tile
-  // rather than in every slab (the first slab's barrier publishes them).
-  for (int lc = tid; lc < ncode; lc += kGemmThreads) {
-    const int col = proj_col(d, tn, lc);  // = h M + c, the gates' index
-    gtab[lc] = (float)gate_q[col] * (float)gate_k[col];
+  // Code columns of the tile: ncode, contiguous in W_phi from code0. Those of
+  // this wave come first in its columns: ncw of them, from place cw of the
+  // tile's; its value columns are W_V's from vw on.
+  const int gpt = d.PCPT > 0 ? BN / d.PGW : 1, col0w = G::WTN * wn;
+  const int ncode = d.PCPT > 0 ? gpt * d.PCPT : max(0, min(BN, d.HM - n0)), code0 = d.PCPT > 0 ? tn * ncode : n0;
+  const int ncw = gpt == 2 ? d.PCPT : min(max(ncode - col0w, 0), G::WTN), cw = gpt == 2 ? wn * d.PCPT : col0w;
+  const int vw = gpt == 2 ? (2 * tn + wn) * d.PVPT
+                          : max(col0w - ncode, 0) + (d.PCPT > 0 ? tn * d.PVPT : max(n0 - d.HM, 0));
+  const int nvw = min(G::WTN, NC - n0 - col0w);  // columns of this wave up to NC (the last tile of the natural order)
+  static_assert(G::WN == 2, "half-tile groups are the two wave columns");
+  const int lrow = lane >> 4, lcol = lane & 15;
+  const bool vec = d.NR % 8 == 0;
+  // ---- values, straight from the accumulators: vt[bh][dd][n] = V_hi, and the
+  // remainder V - V_hi as e4m3 in vlo's tile-major, key-permuted rows. A lane
+  // holds 4 consecutive tokens of one column per 16-row block. Swapping 16-lane
+  // rows between two blocks leaves it 8 consecutive tokens of one of them (a
+  // 16-byte piece of vt, 8 bytes of vlo); with four blocks, swapping 8-lane
+  // halves between the two pairs then puts all 64 tokens of a column into one
+  // store instruction (8 columns x 128 bytes of vt).
+  if (vec && ncode < BN) {
+    constexpr int NP2 = G::FI / 2;  // block pairs
+    static_assert(NP2 == 1 || NP2 == 2, "wave rows of two or four blocks");
+    const bool upper = NP2 == 2 && (lane & 8) != 0;
+    // This lane's 8 tokens start at row tb, position n of batch row b (tb % 8
+    // == 0 and NR % 8 == 0, so they share the batch row and land on 8
+    // consecutive bytes of a vlo row; those past its last token hold zero). In
+    // piece q of a 16-column block they are those of column c0 + 8 q.
+    const int tb = m0 + G::WTM * wm + (upper ? 32 : 0) + 16 * (lrow & 1) + 8 * (lrow >> 1);
+    const int b = tb / d.NR, n = tb - b * d.NR, live = d.N - n;
+    const int c0 = NP2 == 2 ? lcol & 7 : lcol;
+    f16* const dst0 = p.vt + ((int64_t)b * d.D + c0) * d.NP + n;
+    uint8_t* const low0 = p.vlo + (int64_t)b * d.D * d.NP + ((int64_t)(n / 64) * DV + c0) * 64 + vlo_pos(n % 64);
+    unsigned mh[4], ml[2];  // the live tokens' halves and bytes
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mh[e] = live >= 2 * e + 2 ? ~0u : live == 2 * e + 1 ? 0xffffu : 0u;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      ml[e] = live >= 4 * e + 4 ? ~0u : live <= 4 * e ? 0u : ~0u >> (32 - 8 * (live - 4 * e));
+#pragma unroll
+    for (int j = 0; j < G::FJ; ++j) {
+      if (16 * j < ncw || 16 * j >= nvw) continue;  // uniform, like everything up to the lane's column
+      const int vcol = vw + 16 * j - ncw;
+      unsigned hi[NP2][4], lo[NP2][2];  // [pair][dword]: 8 tokens after the swap
+#pragma unroll
+      for (int ip = 0; ip < NP2; ++ip) {
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii) {
+          float vl[4];
+          f16x4 vh;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float x = acc[2 * ip + ii][j][r];
+            asm("" : "+v"(x));  // one evaluation for V_hi and the remainder
+            vh[r] = (f16)x;
+            vl[r] = x - (float)vh[r];
+          }
+          const uint2 u = __builtin_bit_cast(uint2, vh);
+          hi[ip][2 * ii] = u.x;
+          hi[ip][2 * ii + 1] = u.y;
+          lo[ip][ii] = vlo_pack4(vl);
+        }
+        swap16(hi[ip][0], hi[ip][2]);
+        swap16(hi[ip][1], hi[ip][3]);
+        swap16(lo[ip][0], lo[ip][1]);
+      }
+      if constexpr (NP2 == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) swap8(hi[0][e], hi[1][e], upper);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) swap8(lo[0][e], lo[1][e], upper);
+      }
+      f16* const dst = dst0 + (int64_t)vcol * d.NP;
+      uint8_t* const low = low0 + (int64_t)(vcol / DV) * DV * d.NP + vcol % DV * 64;
+      if (tb < TR) {
+#pragma unroll
+        for (int q = 0; q < NP2; ++q) {
+          *reinterpret_cast<uint4*>(dst + (int64_t)8 * q * d.NP) =
+              make_uint4(hi[q][0] & mh[0], hi[q][1] & mh[1], hi[q][2] & mh[2], hi[q][3] & mh[3]);
+          *reinterpret_cast<uint2*>(low + 512 * q) = make_uint2(lo[q][0] & ml[0], lo[q][1] & ml[1]);
+        }
+      }
+    }
+    // the batch row's last group also clears its columns up to NP
+    if (tb < TR && live <= 8 && n + 8 < d.NP) {
+#pragma unroll 1
+      for (int j = 0; j < G::FJ; ++j) {
+        if (16 * j < ncw || 16 * j >= nvw) continue;
+        const int vcol = vw + 16 * j - ncw;
+#pragma unroll 1
+        for (int q = 0; q < NP2; ++q) {
+          f16* const dst = dst0 + (int64_t)(vcol + 8 * q) * d.NP;
+          uint8_t* const low = low0 + (int64_t)(vcol / DV) * DV * d.NP + (vcol % DV + 8 * q) * 64;
+#pragma unroll 1
+          for (int z = 8; n + z < d.NP; z += 8) {  // n and n + z share the 64-key tile
+            *reinterpret_cast<f16x8*>(dst + z) = f16x8{};
+            *reinterpret_cast<uint2*>(low + (vlo_pos((n + z) % 64) - vlo_pos(n % 64))) = make_uint2(0u, 0u);
+          }
+        }
+      }
+    }
   }
-  for (int slab = 0; slab < BM / 64; ++slab) {
-    if (slab > 0) __syncthreads();  // the previous slab has been consumed
-    if (G::WTM * wm / 64 == slab) {  // uniform: this wave row's rows are in the slab
-      const int r0 = G::WTM * wm % 64;
+  // columns that go through LDS: the codes, and the values of rows too short
+  // for whole groups of 8 tokens
+  const int nlds = vec ? ncode : min(BN, NC - n0);
+  if (nlds == 0) return;
+
+  // ---- codes, through LDS: passes of 16 KB rows per wave row, 64 KB rows in
+  // all (KB of the waves' 16-row blocks, as many as the main loop's LDS
+  // holds), so that all the waves write and read in every pass.
+  const int SS = nlds + 4;  // row stride (floats): 16-byte rows, the accumulator stores on 64 distinct banks
+  float* gtab = reinterpret_cast<float*>(smem);  // gate products G = gq gk of the code columns
+  float* stage = gtab + BN;
+  int lk = G::FI >= 4 ? 2 : G::FI >= 2 ? 1 : 0;  // log2 of the blocks per pass
+  while (lk > 0 && BN * 4 + (64 << lk) * SS * 4 > G::kLdsBytes) --lk;
+  const float c1 = 2.0f * d.scale * kLog2e;
+  for (int lc = tid; lc < ncode; lc += kGemmThreads) {
+    gtab[lc] = (float)gate_q[code0 + lc] * (float)gate_k[code0 + lc];  // code0 + lc = h M + c
+  }
+  for (int pass = 0; pass < G::FI >> lk; ++pass) {
+    if (pass > 0) __syncthreads();  // the previous pass has been consumed
 #pragma unroll
-      for (int i = 0; i < G::FI; ++i)
+    for (int i = 0; i < G::FI; ++i) {
+      if (i >> lk != pass) continue;  // uniform
+      float* dst = stage + (64 * (i - (pass << lk)) + 16 * wm + 4 * lrow) * SS + (vec ? cw : col0w) + lcol;
 #pragma unroll
-        for (int j = 0; j < G::FJ; ++j)
+      for (int j = 0; j < G::FJ; ++j)
+        if (16 * j < (vec ? ncw : nvw)) {  // uniform
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            stage[(r0 + 16 * i + 4 * (lane >> 4) + r) * SS + G::WTN * wn + 16 * j + (lane & 15)] = acc[i][j][r];
+          for (int r = 0; r < 4; ++r) dst[r * SS + 16 * j] = acc[i][j][r];
+        }
     }
     __syncthreads();
-    const int row0 = m0 + 64 * slab;
-    // soft-hypercube codes: one (token, head, 8-code chunk) per thread; the
-    // M / 8 chunks of a (token, head) sit on consecutive lanes, which meet in
-    // xor shuffles for the row sums (a head's M columns are contiguous in
-    // both column orders). One thread per (token, head) had left 3/4 of the
-    // workgroup idle at m = 64.
+    // one (token, head, 8-code chunk) per thread; the M / 8 chunks of a
+    // (token, head) sit on consecutive lanes, which meet in xor shuffles for
+    // the row sums (a head's M columns are contiguous in both column orders).
+    // One thread per (token, head) had left 3/4 of the workgroup idle at m = 64.
     constexpr int kChunks = M / 8;
     static_assert(kGemmThreads % kChunks == 0, "a (token, head) never straddles two passes");
-    for (int idx = tid; idx < 8 * ncode; idx += kGemmThreads) {  // 64 rows x (ncode / M heads) x (M / 8 chunks)
+    const int lrows = 6 + lk;  // log2 of the pass's rows
+    for (int idx = tid; idx < (ncode / 8) << lrows; idx += kGemmThreads) {  // rows x heads x (M / 8 chunks)
       const int j = idx % kChunks, item = idx / kChunks;
-      const int hh = item / 64, r = item % 64;
-      const int col0 = proj_col(d, tn, hh * M);
-      const int t = row0 + r;
-      const bool active = t < T;  // the same for every chunk of the item
-      const int h = col0 / M;
-      const int b = t / d.N, n = t - b * d.N;
+      const int hh = item >> lrows, r = item & ((1 << lrows) - 1);
+      const int t = m0 + G::WTM * ((r & 63) >> 4) + 16 * ((pass << lk) + (r >> 6)) + (r & 15);
+      const int h = code0 / M + hh;
+      const int b = t / d.NR, n = t - b * d.NR;
+      const bool active = t < TR && n < d.N;  // the same for every chunk of the item
       const int64_t bhn = (int64_t)(b * d.H + h) * d.N + n;
       const int c8 = 8 * j;
       float sumb = 0.f, tii = 0.f, U = 0.f;
       if (active) {
-        const float* z = stage + r * SS + hh * M + c8;
+        const float* zp = stage + r * SS + hh * M + c8;
+        const float4 za = *reinterpret_cast<const float4*>(zp), zb = *reinterpret_cast<const float4*>(zp + 4);
+        const float z[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
         const float4 ga = *reinterpret_cast<const float4*>(gtab + hh * M + c8);
         const float4 gb = *reinterpret_cast<const float4*>(gtab + hh * M + c8 + 4);
         const float g8[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
@@ -247,62 +377,27 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
       *reinterpret_cast<f16x8*>(p.ka + bhn * CW + M) = f16x8{bh_, bl_, one, one, zero, zero, zero, zero};
       p.tstat[bhn] = make_float4(bias, R, gap, t_ii);
     }
-    // values, transposed: vt[bh][dd][n] = V_hi, and the remainder V - V_hi as
-    // e4m3 in vlo's tile-major, key-permuted rows. One item = one column x 8
-    // consecutive tokens; 8 neighbouring threads cover the slab's 64
-    // consecutive tokens of a column (128 contiguous bytes of vt, one 64-byte
-    // row of vlo), a wave 8 columns.
-    // A thread keeps its group of 8 tokens (tid % 8) and steps over the
-    // tile's value columns [ncode, BN).
-    const int rg = tid & 7, tb = row0 + 8 * rg;
-    if (ncode < BN && tb < T) {
-      const bool vec = d.N % 8 == 0;
+    if (!vec) {  // values one at a time
       const int ntile = d.NP / 64;
-      const int tbb = tb / d.N, tbn = tb - tbb * d.N;  // batch row and position of token tb
-      for (int cc = ncode + (tid >> 3); cc < BN; cc += kGemmThreads / 8) {
-        if (n0 + cc >= NC) break;  // columns past NC only at the end of the tile
-        const int col = proj_col(d, tn, cc);
-        const int vcol = col - d.HM, h = vcol / DV, dd = vcol % DV;
-        const float* src = stage + 8 * rg * SS + cc;
-        if (vec) {
-          // N % 8 == 0 and tb % 8 == 0: the 8 tokens share one batch row and
-          // land on 8 consecutive bytes of a vlo row
-          const int b = tbb, n = tbn;
-          const int64_t bh = (int64_t)(b * d.H + h);
-          f16x8 vh;
-          float vl[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float x = src[e * SS];  // a value read from LDS: one evaluation for V_hi and the remainder
-            vh[e] = (f16)x;
-            vl[e] = x - (float)vh[e];
+      for (int idx = tid; idx < (nlds - ncode) << lrows; idx += kGemmThreads) {
+        const int r = idx & ((1 << lrows) - 1), cc = ncode + (idx >> lrows);
+        const int t = m0 + G::WTM * ((r & 63) >> 4) + 16 * ((pass << lk) + (r >> 6)) + (r & 15);
+        if (t >= TR) continue;
+        const int b = t / d.NR, n = t - b * d.NR;  // NR == N here
+        const int vcol = d.PCPT > 0 ? tn * d.PVPT + cc - ncode : n0 + cc - d.HM, h = vcol / DV, dd = vcol % DV;
+        const int64_t bh = (int64_t)b * d.H + h;
+        const float x = stage[r * SS + cc];
+        const f16 vh = (f16)x;
+        f16* dst = p.vt + (bh * DV + dd) * d.NP + n;
+        uint8_t* low = p.vlo + ((bh * ntile + n / 64) * DV + dd) * 64;
+        dst[0] = vh;
+        const float vl[4] = {x - (float)vh, 0.f, 0.f, 0.f};
+        low[vlo_pos(n % 64)] = (uint8_t)vlo_pack4(vl);
+        if (n == d.N - 1)
+          for (int z = 1; n + z < d.NP; ++z) {
+            dst[z] = (f16)0.f;
+            low[vlo_pos((n + z) % 64)] = 0;
           }
-          f16* dst = p.vt + (bh * DV + dd) * d.NP + n;
-          uint8_t* lrow = p.vlo + ((bh * ntile + n / 64) * DV + dd) * 64;
-          *reinterpret_cast<f16x8*>(dst) = vh;
-          *reinterpret_cast<uint2*>(lrow + vlo_pos(n % 64)) = vlo_pack8(vl);
-          if (n + 8 == d.N)
-            for (int z = 8; n + z < d.NP; z += 8) {
-              *reinterpret_cast<f16x8*>(dst + z) = f16x8{};
-              *reinterpret_cast<uint2*>(lrow + vlo_pos((n + z) % 64)) = make_uint2(0u, 0u);
-            }
-        } else {
-          for (int e = 0; e < 8 && tb + e < T; ++e) {
-            const int t = tb + e, b = t / d.N, n = t - b * d.N;
-            const int64_t bh = (int64_t)(b * d.H + h);
-            const float x = src[e * SS];
-            const f16 vh = (f16)x;
-            f16* dst = p.vt + (bh * DV + dd) * d.NP + n;
-            uint8_t* lrow = p.vlo + ((bh * ntile + n / 64) * DV + dd) * 64;
-            dst[0] = vh;
-            lrow[vlo_pos(n % 64)] = (uint8_t)vlo_code(x - (float)vh);
-            if (n == d.N - 1)
-              for (int z = 1; n + z < d.NP; ++z) {
-                dst[z] = (f16)0.f;
-                lrow[vlo_pos((n + z) % 64)] = 0;
-              }
-          }
-        }
       }
     }
   }
@@ -315,7 +410,7 @@ static hipError_t launch_proj_fwd_t(const Dims& d, const f16* X, const f16* gq, 
   const bool gen = d.proj != kProjSigmoid || d.mask_diag;
 #define MORPHO_PROJ_LAUNCH(BM_, BN_)                                                                       \
   do {                                                                                                     \
-    const dim3 g(gemm_tile_grid((int)((d.T + BM_ - 1) / BM_), (NC + BN_ - 1) / BN_));                      \
+    const dim3 g(gemm_tile_grid((int)((d.TR + BM_ - 1) / BM_), (NC + BN_ - 1) / BN_));                      \
     if (gen)                                                                                               \
       MORPHO_KLAUNCH((proj_fwd_kernel<M, DV, BM_, BN_, true>), g, dim3(kGemmThreads), 0, s, X, gq, gk, d, p);  \
     else                                                                                                   \

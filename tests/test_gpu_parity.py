@@ -262,6 +262,25 @@ def test_projection_tile_128x160(B, N, D, H, causal):
           *oracle(x, params, H, m, 0.8, causal, dout))
 
 
+@pytest.mark.parametrize("B,N,H,m,dv", [
+    (3, 31, 2, 16, 64),      # short rows: unpadded, element stores
+    (3, 33, 2, 32, 64),      # padded to 40, 128-row tiles
+    (5, 197, 3, 64, 64),     # padded to 200: batch rows change inside a tile
+    (2, 71, 4, 16, 32),      # last group of one row of 8 with 7 live tokens
+    (64, 130, 32, 16, 64),   # 256 x 320 tiles
+    (64, 129, 16, 64, 64),   # 256 x 256 tiles, half-tile column groups, one live token in the last group
+    (52, 128, 5, 64, 64),    # heads must not straddle 160-column tiles
+], ids=["N31", "N33", "N197", "N71", "t320", "t256", "H5m64"])
+def test_projection_rows_and_tiles(B, N, H, m, dv):
+    """The projection's padded rows (N % 8 != 0), its tile shapes and column
+    orders against the fp32 oracle."""
+    D = H * dv
+    _say(f"[case] projection rows B={B} N={N} D={D} H={H} m={m}")
+    x, params, dout = make_inputs(B, N, D, H, m, seed=5100 + N)
+    out, lse, grads = run_hip(x, params, H, m, m ** -0.5, False, dout)
+    check(f"projection rows N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, m ** -0.5, False, dout))
+
+
 def test_backward_hi_only_scores_guard():
     """At m = 16 with the sigmoid projection the backward recomputes its
     scores from the fp16 hi codes alone only for heads whose code weights
