@@ -24,7 +24,10 @@ __device__ __forceinline__ float sum8(const f16x8& v) {
 // 16 rows one b128 read phase touches land on distinct bank groups.
 __device__ __forceinline__ int vswz(int r) { return (r ^ (r >> 3)) & 7; }
 
-template <int M, int DV, bool SM = false>
+// Launch shapes (SM), by how many workgroups the problem has (launch_attn_fwd_t).
+constexpr int kFwdRegular = 0, kFwdSmall = 1, kFwdSplit = 2;
+
+template <int M, int DV, int SM = kFwdRegular>
 struct FwdCfg {
   static constexpr int CW = 2 * M + 8;    // code row width
   static constexpr int NCH = M / 8;       // 16-wide code chunks (hi, then lo)
@@ -32,17 +35,23 @@ struct FwdCfg {
   // Each wave owns QB blocks of 32 queries: every K / V fragment read from LDS
   // then feeds QB MFMAs. Two blocks where the registers allow it (m dv <=
   // 1024; at m = 32, dv = 64 two blocks spill).
-  // SM (small problems, fewer than two of the regular workgroups per CU): one
-  // query block per wave, four waves, three workgroups per CU, so the launch
-  // has twice the workgroups and still covers the CUs.
+  // kFwdSmall: one query block per wave, four waves, two or three workgroups per
+  // CU, so the launch has twice the workgroups and still covers the CUs.
+  // kFwdSplit: eight waves per 128 queries, the keys split between two groups of
+  // four: group g takes the tiles t = g (mod 2) through stages of its own, and
+  // the partial sums meet in LDS at the end (the row reference is fixed, so
+  // they just add). A workgroup's chain of tiles is half as long.
   // W4 (m >= 32, dv <= 64, one block per wave): four-wave workgroups, two or
   // three per CU (LDS permitting), rather than one of eight waves; the waves
   // of a CU then wait at independent barriers (B1 N16384 H16 m32 causal:
   // forward -6 %; B16 N2048 H32 m64: -7 %).
   static constexpr int QB2 = (M <= 32 && DV <= 64 && M * DV <= 1024) ? 2 : 1;
-  static constexpr bool SMALL = SM && QB2 == 2;
+  static constexpr bool HASSMALL = QB2 == 2 || (DV == 128 && M <= 32);  // else regular is small already
+  static constexpr bool SMALL = SM != kFwdRegular && HASSMALL;
   static constexpr int QB = SMALL ? 1 : QB2;
   static constexpr bool W4 = QB2 == 1 && M >= 32 && DV <= 64;
+  static constexpr bool HASSPLIT = !(M == 64 && DV == 128);  // two groups' stages fit the LDS
+  static constexpr int KS = SM == kFwdSplit ? 2 : 1;          // groups of WAVES waves
   static constexpr int WAVES = (SMALL || W4) ? 4 : 8 / QB;
   static constexpr int QW = 32 * QB * WAVES;  // 128 or 256 queries per workgroup
   // A stage holds one key tile [KT][CW] (rows in swap23 order within each 32,
@@ -70,9 +79,9 @@ struct FwdCfg {
   // 142 VGPRs), else two.
   static constexpr bool TWO = 2 * STAGE * 2 <= 79 * 1024 && QB == 2;
   static constexpr int W4WG = 2 * STAGE * 2 <= 52 * 1024 ? 3 : 2;
-  static constexpr int WG_PER_CU = W4 ? W4WG : SMALL ? 3 : TWO ? 2 : 1;
-  static constexpr int WAVES_PER_EU = WG_PER_CU * WAVES / 4;
-  static constexpr int LDS_BUDGET = (WG_PER_CU == 3 ? 52 : WG_PER_CU == 2 ? 79 : 158) * 1024;
+  static constexpr int WG_PER_CU = KS == 2 ? 1 : W4 || SMALL ? W4WG : TWO ? 2 : 1;
+  static constexpr int WAVES_PER_EU = WG_PER_CU * KS * WAVES / 4;
+  static constexpr int LDS_BUDGET = (WG_PER_CU == 3 ? 52 : WG_PER_CU == 2 ? 79 : 158 / KS) * 1024;  // of one group
   static constexpr int NSTAGE = 3 * STAGE * 2 <= LDS_BUDGET ? 3 : 2;
   // both 32-key blocks of a tile in flight at once (fits the registers except
   // with the widest codes and values)
@@ -86,7 +95,7 @@ struct FwdCfg {
 // to arrive; one barrier per tile.
 // MAXPASS: key tiles only, track the row max of the exponent (exact path).
 // MD: the diagonal (key == query) is masked.
-template <int M, int DV, bool MAXPASS, bool MD, bool SM>
+template <int M, int DV, bool MAXPASS, bool MD, int SM>
 __device__ __forceinline__ void fwd_pass(const f16* __restrict__ ka, const f16* __restrict__ vt,
                                          const uint8_t* __restrict__ vlo, int64_t rowbase, int64_t vbase,
                                          int N, int NP, int causal, int kend, int q0, int qw0,
@@ -98,8 +107,13 @@ __device__ __forceinline__ void fwd_pass(const f16* __restrict__ ka, const f16* 
   constexpr int QB = C::QB;
   constexpr int NPWX = MAXPASS ? C::NPW_K : C::NPW;
   const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nkt = (kend + C::KT - 1) / C::KT;
+  const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wg % C::WAVES, grp = wg / C::WAVES;  // wave of the group, group
+  // The group's i-th tile is tile KS i + grp of the keys: nkt of them; every
+  // group takes part in nit barriers.
+  const int nall = (kend + C::KT - 1) / C::KT, nit = (nall + C::KS - 1) / C::KS;
+  const int nkt = C::KS == 1 ? nall : (nall - grp + C::KS - 1) / C::KS;
+  smem += grp * (C::NSTAGE * C::STAGE);
 
   // LDS byte address of the stage area (the DMA takes raw LDS addresses)
   const unsigned sbase = (unsigned)(uintptr_t)(__attribute__((address_space(3))) f16*)smem;
@@ -129,7 +143,7 @@ __device__ __forceinline__ void fwd_pass(const f16* __restrict__ ka, const f16* 
   }
   auto issue = [&](int t) {
     const unsigned st = sbase + 2u * (unsigned)((t % C::NSTAGE) * C::STAGE);
-    const int k0 = t * C::KT;
+    const int k0 = (C::KS * t + grp) * C::KT;
     if (k0 + C::KT <= N) {  // uniform: no key row past N
       const f16* kbase = ka + (rowbase + k0) * C::CW;
 #pragma unroll
@@ -299,16 +313,19 @@ __device__ __forceinline__ void fwd_pass(const f16* __restrict__ ka, const f16* 
     __builtin_amdgcn_s_barrier();
   };
 
+  const bool idle = qw0 >= N;  // uniform: a wave past the last query only moves tiles
   int t = 0;
   issue_upto(1);
   if (!MAXPASS) {
     // ---- tiles whose 64 keys are unmasked for every query of the workgroup
     // (with the diagonal masked, the tiles from the workgroup's first query on
     // take the masked path)
-    const int nfull = min(nkt, ((causal || MD) ? q0 : N) / C::KT);
+    const int nfall = min(nall, ((causal || MD) ? q0 : N) / C::KT);
+    const int nfull = C::KS == 1 ? nfall : (nfall - grp + C::KS - 1) / C::KS;
     for (; t < nfull; ++t) {
       publish(t);
       issue_upto(t + C::NSTAGE - 1);
+      if (idle) continue;
       const f16* tile = stage(t);
       if (!C::PIPE) {  // registers too tight for two blocks in flight: one block at a time
         i32x8 p8[QB];
@@ -368,15 +385,15 @@ __device__ __forceinline__ void fwd_pass(const f16* __restrict__ ka, const f16* 
     }
   }
   // ---- remaining tiles (masked ones; all of them in the exact-max pass)
-  for (; t < nkt; ++t) {
+  for (; t < nit; ++t) {
     publish(t);
     issue_upto(t + C::NSTAGE - 1);
-    compute(stage(t), t * C::KT);
+    if (!idle && (C::KS == 1 || t < nkt)) compute(stage(t), (C::KS * t + grp) * C::KT);
   }
 }
 
-template <int M, int DV, bool MD, bool SM>
-__global__ __launch_bounds__((64 * FwdCfg<M, DV, SM>::WAVES))
+template <int M, int DV, bool MD, int SM>
+__global__ __launch_bounds__((64 * FwdCfg<M, DV, SM>::WAVES * FwdCfg<M, DV, SM>::KS))
 __attribute__((amdgpu_waves_per_eu(FwdCfg<M, DV, SM>::WAVES_PER_EU, FwdCfg<M, DV, SM>::WAVES_PER_EU)))
 void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16* __restrict__ vt,
                      const uint8_t* __restrict__ vlo,
@@ -384,9 +401,10 @@ void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16
                      int H, int D, int BH, int causal) {
   using C = FwdCfg<M, DV, SM>;
   constexpr int QB = C::QB;
-  __shared__ __align__(16) f16 smem[C::NSTAGE * C::STAGE];
+  __shared__ __align__(16) f16 smem[C::KS * C::NSTAGE * C::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, scalar
+  const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, scalar
+  const int w = wg % C::WAVES, grp = wg / C::WAVES;         // of the group, group
   const int nqb = (N + C::QW - 1) / C::QW;
   int bh, blk;
   if (!(causal ? xcd_map_lpt(nqb, BH, bh, blk) : xcd_map(nqb, BH, bh, blk))) return;
@@ -437,6 +455,15 @@ void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16
       if (h32 == 0) { qa0[qb][2] = (f16)0.f; qa0[qb][3] = (f16)0.f; }
     }
     fwd_pass<M, DV, true, MD, SM>(ka, vt, vlo, rowbase, vbase, N, NP, causal, kend, q0, qw0, smem, qf, qa0, o, lsum, rmax);
+    if constexpr (C::KS == 2) {  // the other group's maxima
+      __syncthreads();           // every wave is done with the stages
+      float* ex = reinterpret_cast<float*>(smem);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) ex[(wg * QB + qb) * 64 + lane] = rmax[qb];
+      __syncthreads();
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) rmax[qb] = fmaxf(rmax[qb], ex[((wg ^ C::WAVES) * QB + qb) * 64 + lane]);
+    }
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const float m = fmaxf(rmax[qb], __shfl_xor(rmax[qb], 32));
@@ -449,6 +476,27 @@ void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16
   }
   fwd_pass<M, DV, false, MD, SM>(ka, vt, vlo, rowbase, vbase, N, NP, causal, kend, q0, qw0, smem, qf, qaug, o, lsum, rmax);
 
+  if constexpr (C::KS == 2) {
+    static_assert(QB == 1, "one query block per wave in the split shape");
+    constexpr int NR = DV / 2 + 1;  // registers to hand over
+    static_assert(C::WAVES * 64 * NR * 4 <= 2 * C::KS * C::NSTAGE * C::STAGE, "partial sums must fit the stages");
+    float* ex = reinterpret_cast<float*>(smem) + w * (64 * NR) + lane;
+    __syncthreads();  // every wave is done with the stages
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < DV / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[64 * (16 * i + r)] = o[0][i][r];
+      ex[64 * (DV / 2)] = lsum[0];
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int i = 0; i < DV / 32; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[0][i][r] += ex[64 * (16 * i + r)];
+    lsum[0] += ex[64 * (DV / 2)];
+  }
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const int q = qw0 + 32 * qb + l32;
@@ -479,27 +527,39 @@ void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16
   }
 }
 
-template <int M, int DV, bool SM>
+template <int M, int DV, int SM>
 static hipError_t launch_attn_fwd_c(const Dims& d, const ProjBuffers& p, f16* out, float* lse, hipStream_t s) {
   using C = FwdCfg<M, DV, SM>;
-  const dim3 grid(xcd_grid((d.N + C::QW - 1) / C::QW, d.B * d.H));
+  const dim3 grid(xcd_grid((d.N + C::QW - 1) / C::QW, d.B * d.H)), block(64 * C::WAVES * C::KS);
   if (d.mask_diag)
-    MORPHO_KLAUNCH((attn_fwd_kernel<M, DV, true, SM>), grid, dim3(64 * C::WAVES), 0, s, p.qa, p.ka, p.vt, p.vlo,
-                       p.tstat, out, lse, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal);
+    MORPHO_KLAUNCH((attn_fwd_kernel<M, DV, true, SM>), grid, block, 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat, out, lse,
+                   d.N, d.NP, d.H, d.D, d.B * d.H, d.causal);
   else
-    MORPHO_KLAUNCH((attn_fwd_kernel<M, DV, false, SM>), grid, dim3(64 * C::WAVES), 0, s, p.qa, p.ka, p.vt,
-                       p.vlo, p.tstat, out, lse, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal);
+    MORPHO_KLAUNCH((attn_fwd_kernel<M, DV, false, SM>), grid, block, 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat, out, lse,
+                   d.N, d.NP, d.H, d.D, d.B * d.H, d.causal);
   return hipGetLastError();
 }
 
+// Launch shape. The split shape where the chain of tiles of one workgroup, not
+// the work of all of them, takes the time: up to one 128-query workgroup per
+// CU (attn_fwd in us, small or regular -> split, B1 H8 m16 dv64 N1024 15.9 ->
+// 13.3, N2048 causal 28.2 -> 22.7, B1 H16 N2048 31.3 -> 26.4; m64 N2048 causal
+// 39.2 -> 32.8), and to two per CU when the mask makes the last queries' chains
+// twice the mean and a head's chains are many against the heads (B1 H16 causal
+// N3001 42.3 -> 33.6, N4096 59.6 -> 49.4; but B8 H8 N1024 18.9 -> 20.6, and
+// unmasked B1 H16 N4096 90.1 -> 92.5). Small below two regular workgroups per
+// CU (m32 dv128, B1 H8 N2048 causal 54.4 -> 40.9; above that, at two per CU,
+// dv128 N4096 H16 135.6 -> 145.2).
 template <int M, int DV>
 static hipError_t launch_attn_fwd_t(const Dims& d, const ProjBuffers& p, f16* out, float* lse, hipStream_t s) {
-  using C = FwdCfg<M, DV, false>;
-  if constexpr (FwdCfg<M, DV, true>::SMALL) {
-    const int64_t wgs = (int64_t)((d.N + C::QW - 1) / C::QW) * d.B * d.H;
-    if (wgs < 2 * 256) return launch_attn_fwd_c<M, DV, true>(d, p, out, lse, s);
-  }
-  return launch_attn_fwd_c<M, DV, false>(d, p, out, lse, s);
+  using C = FwdCfg<M, DV>;
+  const int64_t bh = (int64_t)d.B * d.H, nq128 = (d.N + 127) / 128;
+  if constexpr (C::HASSPLIT)
+    if (nq128 * bh <= 256 || (d.causal && nq128 * bh <= 512 && nq128 >= bh))
+      return launch_attn_fwd_c<M, DV, kFwdSplit>(d, p, out, lse, s);
+  if constexpr (C::HASSMALL)
+    if ((d.N + C::QW - 1) / C::QW * bh < 2 * 256) return launch_attn_fwd_c<M, DV, kFwdSmall>(d, p, out, lse, s);
+  return launch_attn_fwd_c<M, DV, kFwdRegular>(d, p, out, lse, s);
 }
 
 }  // namespace morpho

@@ -281,6 +281,28 @@ def test_projection_rows_and_tiles(B, N, H, m, dv):
     check(f"projection rows N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, m ** -0.5, False, dout))
 
 
+@pytest.mark.parametrize("B,N,H,m,dv,causal", [
+    (1, 40, 1, 16, 64, False),     # split, one tile: the second group has none
+    (1, 65, 2, 32, 32, True),      # split, a second tile of one key
+    (1, 1000, 3, 16, 32, True),    # split, odd number of tiles
+    (2, 900, 2, 64, 64, False),    # split, ragged
+    (1, 700, 2, 32, 128, True),    # split, wide heads
+    (1, 2500, 20, 16, 64, True),   # split up to two workgroups per CU
+    (5, 900, 8, 16, 128, False),   # small shape of wide heads
+    (9, 300, 16, 32, 128, True),   # small, waves past the last query
+], ids=lambda v: str(v))
+def test_forward_launch_shapes(B, N, H, m, dv, causal):
+    """The split and small launch shapes of the forward against the oracle, on
+    the reference path (default gates) and the exact-maximum path (signed
+    gates; 2 sigma keeps the scores of m = 64 in the fp32 oracle's range)."""
+    for gates in (None, (0.0, 2.0)):
+        _say(f"[case] forward shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} gates={gates}")
+        x, params, dout = make_inputs(B, N, H * dv, H, m, seed=5300 + N, gates=gates)
+        scale = m ** -0.5 if gates is None else 0.5 * m ** -0.5
+        out, lse, grads = run_hip(x, params, H, m, scale, causal, dout)
+        check(f"forward shapes N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, scale, causal, dout))
+
+
 def test_backward_hi_only_scores_guard():
     """At m = 16 with the sigmoid projection the backward recomputes its
     scores from the fp16 hi codes alone only for heads whose code weights
