@@ -542,23 +542,20 @@ static hipError_t launch_attn_fwd_c(const Dims& d, const ProjBuffers& p, f16* ou
   return hipGetLastError();
 }
 
-// Launch shape. The split shape where the chain of tiles of one workgroup, not
-// the work of all of them, takes the time: up to one 128-query workgroup per
-// CU (attn_fwd in us, small or regular -> split, B1 H8 m16 dv64 N1024 15.9 ->
-// 13.3, N2048 causal 28.2 -> 22.7, B1 H16 N2048 31.3 -> 26.4; m64 N2048 causal
-// 39.2 -> 32.8), and to two per CU when the mask makes the last queries' chains
-// twice the mean and a head's chains are many against the heads (B1 H16 causal
-// N3001 42.3 -> 33.6, N4096 59.6 -> 49.4; but B8 H8 N1024 18.9 -> 20.6, and
-// unmasked B1 H16 N4096 90.1 -> 92.5). Small below two regular workgroups per
-// CU (m32 dv128, B1 H8 N2048 causal 54.4 -> 40.9; above that, at two per CU,
+// Launch shape. The split shape where the longest chain of tiles of one
+// workgroup is at least the mean work of a CU (few_long_chains): attn_fwd in us,
+// small or regular -> split, B1 H8 m16 dv64 N1024 15.9 -> 13.3, N2048 causal
+// 28.2 -> 22.7, B1 H16 N2048 31.3 -> 26.4, causal N3001 42.3 -> 33.6, N4096 59.6
+// -> 49.4; m64 B1 H8 N2048 causal 39.2 -> 32.8. Beyond: B8 H8 N1024 causal 18.9 ->
+// 20.6, unmasked B1 H16 N4096 90.1 -> 92.5. Small below two regular workgroups
+// per CU (m32 dv128, B1 H8 N2048 causal 54.4 -> 40.9; above that, at two per CU,
 // dv128 N4096 H16 135.6 -> 145.2).
 template <int M, int DV>
 static hipError_t launch_attn_fwd_t(const Dims& d, const ProjBuffers& p, f16* out, float* lse, hipStream_t s) {
   using C = FwdCfg<M, DV>;
-  const int64_t bh = (int64_t)d.B * d.H, nq128 = (d.N + 127) / 128;
+  const int64_t bh = (int64_t)d.B * d.H;
   if constexpr (C::HASSPLIT)
-    if (nq128 * bh <= 256 || (d.causal && nq128 * bh <= 512 && nq128 >= bh))
-      return launch_attn_fwd_c<M, DV, kFwdSplit>(d, p, out, lse, s);
+    if (few_long_chains(d, 528)) return launch_attn_fwd_c<M, DV, kFwdSplit>(d, p, out, lse, s);
   if constexpr (C::HASSMALL)
     if ((d.N + C::QW - 1) / C::QW * bh < 2 * 256) return launch_attn_fwd_c<M, DV, kFwdSmall>(d, p, out, lse, s);
   return launch_attn_fwd_c<M, DV, kFwdRegular>(d, p, out, lse, s);

@@ -34,6 +34,16 @@ struct Dims {
   int PBN, PGW, PCPT, PVPT;
 };
 
+// Whether the longest chain of 128-token blocks of one 128-token workgroup
+// (n128 of them) is at least the mean work of one of the 256 CUs: BH n128^2 / 256
+// blocks, or BH n128 (n128 + 1) / 512 under the causal mask (`causal_limit` for
+// BH (n128 + 1), about 512). The attention kernels then split each chain
+// between two groups of waves.
+inline bool few_long_chains(const Dims& d, int causal_limit) {
+  const int64_t bh = (int64_t)d.B * d.H, n128 = (d.N + 127) / 128;
+  return d.causal ? bh * (n128 + 1) <= causal_limit : bh * n128 <= 256;
+}
+
 // wt row (position in the projection's column order) of [W_phi | W_V] column c.
 __host__ __device__ inline int proj_row(const Dims& d, int c) {
   if (d.PCPT == 0) return c;

@@ -156,7 +156,9 @@ __device__ __forceinline__ f16x8 tfrag16(const char* tile, int k0, int mn0, int 
   return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int M, int DV>
+// SPLIT: two groups of four waves per 128 keys, taking the query steps in turn
+// (launch_attn_bwd_t says when).
+template <int M, int DV, bool SPLIT = false>
 struct BwdCfg {
   static constexpr int CW = 2 * M + 8;
   static constexpr int NCH = M / 8;             // 16-wide code chunks (hi, then lo)
@@ -183,8 +185,9 @@ struct BwdCfg {
   // per (query, code) of each step to dq, so the atomic count scales with the
   // number of key blocks: at m = 32 and 64 8 waves (256 keys) halve it, at
   // one workgroup (two waves per SIMD) per CU.
-  static constexpr int NW = M >= 32 && DV <= 64 ? 8 : 4;
-  static constexpr int NT = 64 * NW;                      // threads
+  static constexpr int NW = !SPLIT && M >= 32 && DV <= 64 ? 8 : 4;
+  static constexpr int NG = SPLIT ? 2 : 1;                // groups of NW waves (of the same keys)
+  static constexpr int NT = 64 * NW * NG;                 // threads
   static constexpr int KW = 32 * NW;                      // keys per workgroup
   // 16x16 dq tiles of a step, and per wave: when there are fewer tiles than
   // waves (m = 32: 4 tiles, 8 waves) the waves w >= DQTILES have no dq work.
@@ -195,9 +198,13 @@ struct BwdCfg {
   static constexpr int QP = QT * QRB / 1024, OP = QT * ORB / 1024;
   static constexpr int QPW = QP / NW, OPW = (OP + NW - 1) / NW;  // pieces per wave (dO: the first OP % NW waves)
   static_assert(QP % NW == 0, "query pieces must split evenly over the waves");
-  static constexpr int MIN_WG = NW == 4 ? 2 : 1;  // workgroups per CU (launch bound)
+  static constexpr int MIN_WG = NW * NG == 4 ? 2 : 1;  // workgroups per CU (launch bound)
   static constexpr int OOFF = QT * QRB, AOFF = OOFF + QT * ORB;  // bytes
   static constexpr int STAGE = AOFF + 1024;
+  // LDS bytes: two stages and two dS^T tiles per group, the phi tile; whether
+  // the workgroup fits the CU (m = 64, dv = 128 split would spill 73 values)
+  static constexpr int STG = NG * 2 * STAGE, SDS = NG * 2 * KW * SRB, SPK = KW * PRB;
+  static constexpr bool FITS = STG + SDS + SPK <= 160 * 1024 && !(M == 64 && DV == 128);
 };
 
 // Key-side (KV-outer) backward. A workgroup owns KW = 32 NW keys (32 per
@@ -229,11 +236,14 @@ struct BwdCfg {
 // the row sums identical from run to run. A store replaces each atomic one
 // for one, so the tile waits count the same operations (waves without a
 // row-sum tile issue no row-sum store and wait as if they had sent none).
+// SPLIT: group g of the workgroup takes the steps s = g (mod 2), through stages
+// and dS^T tiles of its own; both hold the same keys, and the second group's
+// dk, dcb and dV sums are added to the first's at the end.
 // The body of attn_bwd_kernel for key block kblk of (batch, head) bh. The
-// LDS tiles are the kernel's: stg (2 stages), sdS (dS^T of the whole
-// workgroup, two buffers of KW rows = keys) and sPk (phi_hi of the
-// workgroup's keys, row = key).
-template <int M, int DV, bool MD, bool HILO, bool DET>
+// LDS tiles are the kernel's: per group 2 stages and dS^T of the whole group
+// (two buffers of KW rows = keys), then sPk (phi_hi of the workgroup's keys,
+// row = key).
+template <int M, int DV, bool MD, bool HILO, bool DET, bool SPLIT>
 __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, int bh, int kblk,
                                               const f16* __restrict__ qa, const f16* __restrict__ ka,
                                               const f16* __restrict__ vt, const f16* __restrict__ aug,
@@ -241,11 +251,17 @@ __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, 
                                               float* __restrict__ dk, float* __restrict__ dcb, float* __restrict__ dr,
                                               f16* __restrict__ dzv, int N, int NP, int H, int D, int HM, int BH,
                                               int causal) {
-  using C = BwdCfg<M, DV>;
+  using C = BwdCfg<M, DV, SPLIT>;
+  const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, scalar
+  const int w = wv % C::NW, grp = wv / C::NW;               // of the group, group
+  char* const stg0 = stg;
+  if constexpr (C::NG == 2) {  // the group's own
+    stg += grp * (C::STG / 2);
+    sdS0 += grp * (C::SDS / 2);
+  }
   auto sdS = [&](int par) { return sdS0 + par * (C::KW * C::SRB); };
 
-  const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, scalar
   const int nkb = (N + C::KW - 1) / C::KW;
   const int k0 = kblk * C::KW;  // causal: low key blocks see the most queries; they start first
   const int kw0 = k0 + 32 * w;
@@ -299,17 +315,19 @@ __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, 
   float dcb_acc = 0.f;  // DCB_VALU: this lane's share of dcb[key]
 
   const int qstart = causal ? k0 : 0;
-  const int nsteps = qstart < N ? (N - qstart + C::QT - 1) / C::QT : 0;
+  const int nall = qstart < N ? (N - qstart + C::QT - 1) / C::QT : 0;
+  // the group's own steps: its i-th is step NG i + grp of the block's
+  const int nsteps = C::NG == 1 ? nall : (nall - grp + C::NG - 1) / C::NG;
   // Query tile of step st. Without the causal mask every key block visits all
   // query tiles; block kblk starts kblk / nkb of the way round, so the blocks
   // of a head add their dq and row-sum atomics to different rows at any one
   // time (in lockstep they contended for the same rows' memory-side atomics:
   // C5 attn_bwd 4.06 -> 3.71 ms, C2 0.052 -> 0.048 ms). Causal blocks already
   // start at their own keys.
-  const int qrot = causal ? 0 : (int)(((int64_t)kblk * nsteps) / nkb);
+  const int qrot = causal ? 0 : (int)(((int64_t)kblk * nall) / nkb);
   auto qstep = [&](int st) {
-    const int r = st + qrot;
-    return qstart + (r < nsteps ? r : r - nsteps) * C::QT;
+    const int r = C::NG * st + (C::NG == 1 ? 0 : grp) + qrot;
+    return qstart + (r < nall ? r : r - nall) * C::QT;
   };
 
   // ---- DMA of a step's tiles. Per-lane byte offsets from the step's bases
@@ -717,6 +735,45 @@ __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, 
     rowsum(nsteps - 1);
     dq_finish(nsteps - 1);
   }
+  if constexpr (C::NG == 2) {
+    // the second group's sums through LDS; a group with one step fewer first
+    // makes up for its barriers (nsteps + 1 of them, or none without steps)
+    const int most = (nall + 1) / 2;
+    for (int b = nsteps > 0 ? nsteps + 1 : 0; b < (most > 0 ? most + 1 : 0); ++b) __builtin_amdgcn_s_barrier();
+    static_assert(64 * C::NW * (DV / 2) * 4 <= C::STG && 64 * C::NW * (16 * C::MB + 1) * 4 <= C::STG,
+                  "partial sums must fit the stages");
+    float* ex = reinterpret_cast<float*>(stg0) + tid % (64 * C::NW);
+    constexpr int RS = 64 * C::NW;  // floats per register handed over
+    __syncthreads();  // every wave is done with the stages
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < DV / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[RS * (16 * i + r)] = dva[i][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < DV / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dva[i][r] += ex[RS * (16 * i + r)];
+    }
+    __syncthreads();
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < C::MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[RS * (16 * i + r)] = dka[i][r];
+      ex[RS * 16 * C::MB] = dcb_acc;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int i = 0; i < C::MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dka[i][r] += ex[RS * (16 * i + r)];
+    dcb_acc += ex[RS * 16 * C::MB];
+  }
 
   // ---- epilogue: dk, dcb (fp32, per key) and dV (fp16 into the dZ|dV buffer)
   const float dcb_sum = dcb_acc + __shfl_xor(dcb_acc, 32);  // lanes l, l + 32: the same key
@@ -757,16 +814,16 @@ constexpr float kHiOnlyWeight = 32.f;
 // where the head's code weights are within kHiOnlyWeight, from hi and lo
 // elsewhere (the decision is the workgroup's; both bodies share the LDS
 // tiles). Without HIOK always from hi and lo.
-template <int M, int DV, bool MD, bool HIOK, bool DET>
-__global__ __launch_bounds__((BwdCfg<M, DV>::NT), (BwdCfg<M, DV>::MIN_WG)) void attn_bwd_kernel(
+template <int M, int DV, bool MD, bool HIOK, bool DET, bool SPLIT>
+__global__ __launch_bounds__((BwdCfg<M, DV, SPLIT>::NT), (BwdCfg<M, DV, SPLIT>::MIN_WG)) void attn_bwd_kernel(
     const f16* __restrict__ qa, const f16* __restrict__ ka, const f16* __restrict__ vt, const f16* __restrict__ aug,
     const f16* __restrict__ grad_out, float* __restrict__ dq, float* __restrict__ dk, float* __restrict__ dcb,
     float* __restrict__ dr, f16* __restrict__ dzv, const f16* __restrict__ gate_q, const f16* __restrict__ gate_k,
     float scale, int N, int NP, int H, int D, int HM, int BH, int causal) {
-  using C = BwdCfg<M, DV>;
-  __shared__ __align__(16) char stg[2 * C::STAGE];
-  __shared__ __align__(16) char sdS[2 * C::KW * C::SRB];
-  __shared__ __align__(16) char sPk[C::KW * C::PRB];
+  using C = BwdCfg<M, DV, SPLIT>;
+  __shared__ __align__(16) char stg[C::STG];
+  __shared__ __align__(16) char sdS[C::SDS];
+  __shared__ __align__(16) char sPk[C::SPK];
   int bh, kblk;
   const int nkb = (N + C::KW - 1) / C::KW;
   if (!(causal ? xcd_map_lpt(nkb, BH, bh, kblk) : xcd_map(nkb, BH, bh, kblk))) return;
@@ -779,26 +836,26 @@ __global__ __launch_bounds__((BwdCfg<M, DV>::NT), (BwdCfg<M, DV>::MIN_WG)) void 
     hilo = __builtin_amdgcn_readfirstlane(fabsf(scale) * wsum > kHiOnlyWeight ? 1 : 0) != 0;
   }
   if (hilo)
-    attn_bwd_body<M, DV, MD, true, DET>(stg, sdS, sPk, bh, kblk, qa, ka, vt, aug, grad_out, dq, dk, dcb, dr, dzv, N,
+    attn_bwd_body<M, DV, MD, true, DET, SPLIT>(stg, sdS, sPk, bh, kblk, qa, ka, vt, aug, grad_out, dq, dk, dcb, dr, dzv, N,
                                         NP, H, D, HM, BH, causal);
   else if constexpr (HIOK)
-    attn_bwd_body<M, DV, MD, false, DET>(stg, sdS, sPk, bh, kblk, qa, ka, vt, aug, grad_out, dq, dk, dcb, dr, dzv, N,
+    attn_bwd_body<M, DV, MD, false, DET, SPLIT>(stg, sdS, sPk, bh, kblk, qa, ka, vt, aug, grad_out, dq, dk, dcb, dr, dzv, N,
                                          NP, H, D, HM, BH, causal);
 }
 
-template <int M, int DV, bool HIOK, bool DET>
+template <int M, int DV, bool HIOK, bool DET, bool SPLIT>
 static hipError_t launch_attn_bwd_c(const Dims& d, const ProjBuffers& p, const f16* grad_out, const f16* gate_q,
                                     const f16* gate_k, const BwdBuffers& g, hipStream_t s) {
-  using C = BwdCfg<M, DV>;
+  using C = BwdCfg<M, DV, SPLIT>;
   const dim3 grid(xcd_grid((d.N + C::KW - 1) / C::KW, d.B * d.H));
   float* const dq = DET ? g.dqpart : g.dq;
   float* const dr = DET ? g.drpart : g.dr;
   if (d.mask_diag)
-    MORPHO_KLAUNCH((attn_bwd_kernel<M, DV, true, HIOK, DET>), grid, dim3(C::NT), 0, s, p.qa, p.ka, p.vt, g.aug,
+    MORPHO_KLAUNCH((attn_bwd_kernel<M, DV, true, HIOK, DET, SPLIT>), grid, dim3(C::NT), 0, s, p.qa, p.ka, p.vt, g.aug,
                    grad_out, dq, g.dk, g.dcb, dr, g.dzv, gate_q, gate_k, d.scale, d.N, d.NP, d.H, d.D, d.HM,
                    d.B * d.H, d.causal);
   else
-    MORPHO_KLAUNCH((attn_bwd_kernel<M, DV, false, HIOK, DET>), grid, dim3(C::NT), 0, s, p.qa, p.ka, p.vt, g.aug,
+    MORPHO_KLAUNCH((attn_bwd_kernel<M, DV, false, HIOK, DET, SPLIT>), grid, dim3(C::NT), 0, s, p.qa, p.ka, p.vt, g.aug,
                    grad_out, dq, g.dk, g.dcb, dr, g.dzv, gate_q, gate_k, d.scale, d.N, d.NP, d.H, d.D, d.HM,
                    d.B * d.H, d.causal);
   return hipGetLastError();
@@ -809,9 +866,21 @@ static hipError_t launch_attn_bwd_h(const Dims& d, const ProjBuffers& p, const f
                                     const f16* gate_k, const BwdBuffers& g, hipStream_t s) {
   if (d.det) {
     if (!g.dqpart || !g.drpart) return hipErrorInvalidValue;
-    return launch_attn_bwd_c<M, DV, HIOK, true>(d, p, grad_out, gate_q, gate_k, g, s);
+    return launch_attn_bwd_c<M, DV, HIOK, true, false>(d, p, grad_out, gate_q, gate_k, g, s);
   }
-  return launch_attn_bwd_c<M, DV, HIOK, false>(d, p, grad_out, gate_q, gate_k, g, s);
+  // The split shape where the longest chain of steps of one workgroup is at
+  // least the mean work of a CU (few_long_chains). attn_bwd in us, regular ->
+  // split: B1 H8 m32 dv64 N1024 43.7 -> 26.8, N2048 causal 81.3 -> 47.9, B1 H16
+  // causal N3001 m16 70.6 -> 52.3, m32 117 -> 87, B1 H16 N2048 m16 51.7 -> 41.9,
+  // m64 N2048 causal H8 116 -> 78, B2 H8 N1001 m32 dv128 54.8 -> 42.6. Beyond,
+  // the regular shape: unmasked B1 H16 N4096 m32 177 -> 217, causal B8 H8 N1024
+  // 55.3 -> 56.4 (dv 128); at m >= 32 it has eight waves on 256 keys and half
+  // the dq atomics (B1 H16 N4096 causal m64 225 -> 229, m32 157 -> 115), and
+  // two key blocks are too few steps (B8 H12 N197 m64 28.0 -> 30.4).
+  if constexpr (BwdCfg<M, DV, true>::FITS)
+    if (d.N > 256 && few_long_chains(d, M == 64 ? 420 : 528))
+      return launch_attn_bwd_c<M, DV, HIOK, false, true>(d, p, grad_out, gate_q, gate_k, g, s);
+  return launch_attn_bwd_c<M, DV, HIOK, false, false>(d, p, grad_out, gate_q, gate_k, g, s);
 }
 
 // The hi-only scores are possible at m = 16 with the sigmoid projection

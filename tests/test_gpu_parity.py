@@ -290,17 +290,23 @@ def test_projection_rows_and_tiles(B, N, H, m, dv):
     (1, 2500, 20, 16, 64, True),   # split up to two workgroups per CU
     (5, 900, 8, 16, 128, False),   # small shape of wide heads
     (9, 300, 16, 32, 128, True),   # small, waves past the last query
+    (2, 257, 2, 16, 64, True),     # split backward: three key blocks, one key in the last
+    (1, 288, 3, 64, 32, False),    # split backward, nine steps: one more for the first group
+    (1, 1100, 2, 64, 64, True),    # split backward, two dq tiles per wave
+    (44, 300, 2, 32, 64, True),    # regular backward, eight waves on 256 keys
+    (44, 300, 2, 64, 32, True),
+    (44, 300, 2, 64, 64, False),
 ], ids=lambda v: str(v))
-def test_forward_launch_shapes(B, N, H, m, dv, causal):
-    """The split and small launch shapes of the forward against the oracle, on
-    the reference path (default gates) and the exact-maximum path (signed
+def test_launch_shapes(B, N, H, m, dv, causal):
+    """The split and small launch shapes of the forward and the split shape of
+    the backward against the oracle, on the reference path (default gates) and the exact-maximum path (signed
     gates; 2 sigma keeps the scores of m = 64 in the fp32 oracle's range)."""
     for gates in (None, (0.0, 2.0)):
-        _say(f"[case] forward shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} gates={gates}")
+        _say(f"[case] launch shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} gates={gates}")
         x, params, dout = make_inputs(B, N, H * dv, H, m, seed=5300 + N, gates=gates)
         scale = m ** -0.5 if gates is None else 0.5 * m ** -0.5
         out, lse, grads = run_hip(x, params, H, m, scale, causal, dout)
-        check(f"forward shapes N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, scale, causal, dout))
+        check(f"launch shapes N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, scale, causal, dout))
 
 
 def test_backward_hi_only_scores_guard():
