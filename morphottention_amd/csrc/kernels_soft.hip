@@ -1191,12 +1191,15 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
                         phib[t][kc], a);
         }
         // rows: queries 16 qt + 4 (lane / 16) + r; column: code 16 ct + lane % 16.
-        // Always issued (a fixed count per step: the stage waits count on
-        // it); rows past N add 0 to row N - 1.
+        // Issued by some lane whatever the rows (a fixed count per step: the
+        // stage waits count on it); rows past N add 0 to the row one step back,
+        // each its own. With fewer rows than a step there is one step, and no
+        // wait that counts its atomics.
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int qq = qs + 16 * qt + 4 * (lane >> 4) + r;
-          unsafeAtomicAdd(dq + (rowbase + min(qq, N - 1)) * M + 16 * ct + (lane & 15), qq < N ? a[r] : 0.f);
+          if (qq < N || N >= QT)
+            unsafeAtomicAdd(dq + (rowbase + (qq < N ? qq : qq - QT)) * M + 16 * ct + (lane & 15), qq < N ? a[r] : 0.f);
         }
       }
     }
