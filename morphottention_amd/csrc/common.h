@@ -241,24 +241,47 @@ __device__ __forceinline__ int sswz(int r) {
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (id % 8), each with
-// its own L2. Map a 1-D grid of 8 * ceil(BH / 8) * nblk workgroups so that all
-// blocks of one (batch, head) run on the same XCD and share its L2: XCD x
-// serves heads x, x + 8, ... in turn. Returns false for the padding slots.
+// its own L2. Map a 1-D grid (xcd_grid) so that all blocks of one (batch, head)
+// run on the same XCD and share its L2: XCD x serves heads x, x + 8, ... in
+// turn. Where that would leave a tenth of the XCDs' time idle (few heads that 8
+// does not divide: three heads leave five XCDs without work), the head-major
+// list of blocks is cut into 8 equal runs instead, so only the heads at a cut
+// share two XCDs. attn_fwd / attn_bwd in us, whole heads -> runs: B1 N8192 H3
+// m16 157 -> 76 / 246 -> 121, m64 260 -> 116 / 604 -> 362, B1 N8192 H12 m16
+// causal 157 -> 140 / 251 -> 214, 28 heads N4096 causal 84.7 -> 79.2 / 134 ->
+// 121; but 60 heads N4000 causal (7 % idle) 145 -> 151. Returns false for the
+// padding slots.
+__host__ __device__ __forceinline__ bool xcd_whole_heads(int BH) { return 10 * (-BH & 7) <= BH; }
 __device__ __forceinline__ bool xcd_map(int nblk, int BH, int& bh, int& blk) {
   const int i = blockIdx.x, xcd = i & 7, slot = i >> 3;
+  if (!xcd_whole_heads(BH)) {
+    const int k = xcd * ((BH * nblk + 7) / 8) + slot;
+    bh = k / nblk;
+    blk = k % nblk;
+    return bh < BH;
+  }
   bh = 8 * (slot / nblk) + xcd;
   blk = slot % nblk;
   return bh < BH;
 }
 // Same XCD per head, but block-major within an XCD: for causal problems block
 // 0 is the longest, so all heads' long blocks start first (longest processing
-// time first), and the short ones fill in at the end.
+// time first), and the short ones fill in at the end. With few heads that 8
+// does not divide, the blocks of all heads are dealt to the XCDs in turn.
 __device__ __forceinline__ bool xcd_map_lpt(int nblk, int BH, int& bh, int& blk) {
   const int i = blockIdx.x, xcd = i & 7, slot = i >> 3, hx = (BH + 7) / 8;
+  if (!xcd_whole_heads(BH)) {
+    bh = i % BH;
+    blk = i / BH;
+    return blk < nblk;
+  }
   bh = 8 * (slot % hx) + xcd;
   blk = slot / hx;
   return bh < BH;
 }
-__host__ inline unsigned xcd_grid(int nblk, int BH) { return 8u * (unsigned)((BH + 7) / 8) * (unsigned)nblk; }
+__host__ inline unsigned xcd_grid(int nblk, int BH) {
+  return 8u * (xcd_whole_heads(BH) ? (unsigned)((BH + 7) / 8) * (unsigned)nblk
+                                   : ((unsigned)BH * (unsigned)nblk + 7u) / 8u);
+}
 
 }  // namespace morpho
