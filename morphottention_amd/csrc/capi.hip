@@ -126,15 +126,25 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
     const int ntn = NC / bn;
     return d.HM % ntn == 0 && d.D % ntn == 0 && (d.HM / ntn) % d.M == 0 && (d.D / ntn) % 16 == 0;
   };
+  d.PBM = 256;
   d.PBN = NC % 320 == 0 ? 320 : 256;
-  if (((d.TR + 255) / 256) * ((NC + d.PBN - 1) / d.PBN) < 256) {
-    const int64_t rows = (d.TR + 127) / 128;
+  const int64_t rows = (d.TR + 127) / 128, big = (d.TR + 255) / 256 * ((NC + d.PBN - 1) / d.PBN);
+  if (big >= 256) {
+    // 128 x 256 tiles (one per CU, three stages) where their rounds, 0.58 of a
+    // 256 x 256 round each, are the shorter: a last round of few tiles costs
+    // half. proj_fwd in us, 256 -> 128 rows: B64 N197 D768 H12 m64 (300 tiles)
+    // 81 -> 69, B64 N256 78 -> 73, B1 N16384 D1024 H16 m32 92 -> 86, B4 N4096
+    // D1024 H8 m16 dv128 74 -> 68; the 320-wide tile has no such half.
+    const int64_t half = rows * ((NC + 255) / 256);
+    if (d.PBN == 256 && 100 * ((big + 255) / 256) > 58 * ((half + 255) / 256)) d.PBM = 128;
+  } else {
     int64_t best = -1;
     for (const int bn : {160, 128}) {
       if (NC % bn || (bn % d.M && !whole_heads(bn))) continue;
       const int64_t cost = (rows * (NC / bn) + 255) / 256 * bn;
       if (best < 0 || cost < best) {
         best = cost;
+        d.PBM = 128;
         d.PBN = bn;
       }
     }

@@ -31,7 +31,7 @@ struct Dims {
   // holds code columns [g PCPT, (g+1) PCPT) then value columns [g PVPT, (g+1)
   // PVPT), so every tile (and, with half tiles, every wave) does the same
   // epilogue work; PCPT == 0 keeps the natural order [W_phi | W_V].
-  int PBN, PGW, PCPT, PVPT;
+  int PBM, PBN, PGW, PCPT, PVPT;  // PBM: tile rows
 };
 
 // Whether the longest chain of 128-token blocks of one 128-token workgroup

@@ -72,7 +72,10 @@ hipError_t launch_transpose_weights(const Dims& d, const f16* W_phi, const f16* 
 // H*M + D columns (e.g. 1280 at B4 N4096 D1024 H16 m16, which makes the grid
 // exactly one round of 256 tiles), 256 x 256 otherwise, and 128 x 128 when
 // the large tiles would leave most CUs idle (few tokens: B8 N1024 D512 H8 m16
-// has 64 large tiles, 320 small ones).
+// has 64 large tiles, 320 small ones); between them 128 x 256, where half the
+// tile halves the loss of the last round (make_dims). The 128 x 128 and 128 x
+// 160 tiles run two to a CU with two stages each; with four stages, one to a
+// CU, they gained 1 us or lost up to 9 (B64 N128 D1024 H16 m16 31 -> 40).
 //
 // Epilogue: the values leave straight from the accumulators (lane swaps
 // assemble 16-byte stores), the codes through LDS, and no wave waits for
@@ -85,8 +88,8 @@ hipError_t launch_transpose_weights(const Dims& d, const f16* W_phi, const f16* 
 // H12 m64 142 -> 80, B3 N1500 D1024 H8 m32 42.7 -> 23.8, B64 N128 D1024 H16 m16
 // 40.0 -> 31.0, B64 N1024 D768 H12 m64 256 -> 246, B4 N4096 D1024 H16 m16 55.4
 // -> 56.0 (the first two mostly from the padded rows, make_dims).
-template <int BM, int BN>
-using ProjGemm = Gemm<BM, BN, 4, true, true, 64, 2>;
+template <int BM, int BN, int STAGES>
+using ProjGemm = Gemm<BM, BN, 4, true, true, 64, STAGES>;
 
 // e4m3 byte(s) of V_lo * 2^kVloExp, clamped to the format's range (e4m3 has
 // no infinity: an overflowing conversion gives NaN) and rounded toward zero:
@@ -134,11 +137,11 @@ struct TokenRows {
 
 // GEN: a cube projection other than the sigmoid, or the masked diagonal (the
 // variants take the projection from d.proj and the exact row maximum)
-template <int M, int DV, int BM, int BN, bool GEN>
+template <int M, int DV, int BM, int BN, int STAGES, bool GEN>
 __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __restrict__ X,
                                                                const f16* __restrict__ gate_q,
                                                                const f16* __restrict__ gate_k, Dims d, ProjBuffers p) {
-  using G = ProjGemm<BM, BN>;
+  using G = ProjGemm<BM, BN, STAGES>;
   static_assert(64 * (BN + 4) * 4 + BN * 4 <= G::kLdsBytes, "a pass of 64 code rows and the gates must fit the LDS");
   static_assert(G::WTM == 16 * G::FI && G::FI % 2 == 0 && G::WTM * 4 == BM, "four wave rows of whole block pairs");
   __shared__ __align__(16) char smem[G::kLdsBytes];
@@ -408,22 +411,24 @@ static hipError_t launch_proj_fwd_t(const Dims& d, const f16* X, const f16* gq, 
                                     hipStream_t s) {
   const int NC = d.HM + d.D;
   const bool gen = d.proj != kProjSigmoid || d.mask_diag;
-#define MORPHO_PROJ_LAUNCH(BM_, BN_)                                                                       \
-  do {                                                                                                     \
-    const dim3 g(gemm_tile_grid((int)((d.TR + BM_ - 1) / BM_), (NC + BN_ - 1) / BN_));                      \
-    if (gen)                                                                                               \
-      MORPHO_KLAUNCH((proj_fwd_kernel<M, DV, BM_, BN_, true>), g, dim3(kGemmThreads), 0, s, X, gq, gk, d, p);  \
-    else                                                                                                   \
-      MORPHO_KLAUNCH((proj_fwd_kernel<M, DV, BM_, BN_, false>), g, dim3(kGemmThreads), 0, s, X, gq, gk, d, p); \
+#define MORPHO_PROJ_LAUNCH(BM_, BN_, ST_)                                                                      \
+  do {                                                                                                         \
+    const dim3 g(gemm_tile_grid((int)((d.TR + BM_ - 1) / BM_), (NC + BN_ - 1) / BN_));                         \
+    if (gen)                                                                                                   \
+      MORPHO_KLAUNCH((proj_fwd_kernel<M, DV, BM_, BN_, ST_, true>), g, dim3(kGemmThreads), 0, s, X, gq, gk, d, p);  \
+    else                                                                                                       \
+      MORPHO_KLAUNCH((proj_fwd_kernel<M, DV, BM_, BN_, ST_, false>), g, dim3(kGemmThreads), 0, s, X, gq, gk, d, p); \
   } while (0)
-  if (d.PBN == 320)
-    MORPHO_PROJ_LAUNCH(256, 320);
+  if (d.PBM == 256 && d.PBN == 320)
+    MORPHO_PROJ_LAUNCH(256, 320, 2);
+  else if (d.PBM == 256)
+    MORPHO_PROJ_LAUNCH(256, 256, 2);
+  else if (d.PBN == 256)  // one workgroup per CU: room for a third stage
+    MORPHO_PROJ_LAUNCH(128, 256, 3);
   else if (d.PBN == 160)
-    MORPHO_PROJ_LAUNCH(128, 160);
-  else if (d.PBN == 128)
-    MORPHO_PROJ_LAUNCH(128, 128);
+    MORPHO_PROJ_LAUNCH(128, 160, 2);
   else
-    MORPHO_PROJ_LAUNCH(256, 256);
+    MORPHO_PROJ_LAUNCH(128, 128, 2);
 #undef MORPHO_PROJ_LAUNCH
   return hipGetLastError();
 }
@@ -569,9 +574,11 @@ struct BwdTiles {
 // workgroup), the most pieces p per dW tile that still fit the round,
 // scored by the longer of the two kinds: g kx against ceil(kw / p) k-steps
 // (plus one step of epilogue per dX tile or piece). When the dW tiles alone
-// fill the round, every workgroup takes one tile over several rounds. A type-A workgroup's dX
-// tiles come from the row panels tr = 8 i + xcd, as before, so a panel of
-// dZ|dV is read into one L2.
+// fill the round, every workgroup takes one tile over several rounds. The dX
+// tiles, row panel by row panel, are dealt to the XCDs in 8 equal runs, so all
+// but the panels at a cut are read into one L2 (whole panels per XCD left
+// workgroups without a tile: 18 of 168 at B64 N197 D768 H12 m64, where the dW
+// pieces then took 50 k-steps instead of 40).
 static BwdGemmPlan plan_for(const Dims& d, int bt, int slots, int64_t& cost) {
   BwdGemmPlan P;
   const int NC = d.HM + d.D, T = (int)d.T;
@@ -583,7 +590,7 @@ static BwdGemmPlan plan_for(const Dims& d, int bt, int slots, int64_t& cost) {
   P.ntn_w = (NC + bt - 1) / bt;
   P.tiles_w = ((d.D + bt - 1) / bt) * P.ntn_w;
   P.kw = (T + 63) / 64;
-  const int per_xcd = ((ntm_x + 7) / 8) * P.ntn_x;  // dX tiles of one XCD
+  const int per_xcd = (P.n_dx + 7) / 8;  // dX tiles of one XCD
   cost = INT64_MAX;
   P.g = per_xcd;
   P.n_a = 8;
@@ -604,6 +611,9 @@ static BwdGemmPlan plan_for(const Dims& d, int bt, int slots, int64_t& cost) {
     }
     if (ca > cost) break;  // g kx only grows from here
   }
+  // no more pieces than the cost needs: each is a partial to write and add (B3
+  // N1500 D1024 H8 m32 dv128: 9 -> 4 pieces)
+  while (cost != INT64_MAX && P.p > 1 && (P.kw + P.p - 2) / (P.p - 1) + 1 <= cost) --P.p;
   if (cost == INT64_MAX) {
     // dW tiles alone fill the round: one dX tile or one whole dW tile per
     // workgroup over several rounds (the dispatcher balances them)
@@ -647,14 +657,13 @@ __global__ __launch_bounds__(kGemmThreads) void bwd_gemm_kernel(Dims d, BwdBuffe
   const int id = blockIdx.x;
 
   if (id < P.n_a) {
-    // ---- g dX tiles: local tiles s g .. s g + g - 1 of XCD xcd, i.e. row
-    // panel tr = 8 (L / ntn_x) + xcd, column tile L % ntn_x
-    const int xcd = id & 7, slot = id >> 3;
-    const int ntm = (T + BT - 1) / BT;
+    // ---- g dX tiles: tiles s g .. s g + g - 1 of XCD xcd's run of the row
+    // panels' column tiles
+    const int xcd = id & 7, slot = id >> 3, run = (P.n_dx + 7) / 8;
     for (int q = 0; q < P.g; ++q) {
-      const int L = slot * P.g + q;
-      const int tm = 8 * (L / P.ntn_x) + xcd, tn = L % P.ntn_x;
-      if (tm >= ntm) break;  // uniform
+      const int o = slot * P.g + q, L = xcd * run + o;
+      const int tm = L / P.ntn_x, tn = L % P.ntn_x;
+      if (o >= run || L >= P.n_dx) break;  // uniform
       if (q > 0) __syncthreads();  // the previous tile's slab reads are done before the stages refill
       const int m0 = tm * BT, n0 = tn * BT;
       f32x4 acc[DxGemm::FI][DxGemm::FJ];
