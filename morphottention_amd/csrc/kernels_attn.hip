@@ -525,8 +525,8 @@ __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, 
     const int j = lane & 3;
     const float rsum = j == 0 ? racc[0] : j == 1 ? racc[1] : j == 2 ? racc[2] : racc[3];
     const int qq = qs + rs_row;
-    if ((lane & 15) < 4 && (qq < N || N >= C::QT))
-      unsafeAtomicAdd(&dr[2 * (rowbase + (qq < N ? qq : qq - C::QT))], rs_wave && qq < N ? rsum : 0.f);
+    if ((lane & 15) < 4)
+      unsafeAtomicAdd(&dr[2 * (rowbase + (qq < N ? qq : max(qq - C::QT, 0)))], rs_wave && qq < N ? rsum : 0.f);
   };
   auto dq_finish = [&](int st) {
     if (!dq_wave) return;
@@ -559,14 +559,13 @@ __device__ __forceinline__ void attn_bwd_body(char* stg, char* sdS0, char* sPk, 
         } else {
           const int qq = qs + 16 * qt + 4 * (lane >> 4) + r;
           const bool ok = qq < N;
-          // Issued by some lane whatever the rows (a fixed count per step):
-          // rows past N add 0 to the row one step back, each its own. (All of
-          // them on row N - 1, their atomics queued up on its addresses: B20
-          // N200 H12 m16 causal 33.7 us, now 13.8.) With fewer rows than a
-          // step there is one step, and no wait that counts its atomics.
-          if (ok || N >= C::QT)
-            unsafeAtomicAdd(dq + (rowbase + (ok ? qq : qq - C::QT)) * M + 16 * ((w + C::NW * t) / (C::QT / 16)) + (lane & 15),
-                            ok ? acc[r] : 0.f);
+          // Always issued (a fixed count per step); rows past N add 0 to the
+          // row one step back, each its own. (All of them on row N - 1, their
+          // atomics queued up on its addresses: B20 N200 H12 m16 causal 33.7
+          // us, now 13.8.)
+          unsafeAtomicAdd(dq + (rowbase + (ok ? qq : max(qq - C::QT, 0))) * M +
+                              16 * ((w + C::NW * t) / (C::QT / 16)) + (lane & 15),
+                          ok ? acc[r] : 0.f);
         }
       }
     }

@@ -1191,20 +1191,14 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
                         phib[t][kc], a);
         }
         // rows: queries 16 qt + 4 (lane / 16) + r; column: code 16 ct + lane % 16.
-        // A fixed count per step (the stage waits count on it): in the ragged
-        // step rows past N add 0 to the row one step back, each its own. With
-        // fewer rows than a step there is one step, and no wait that counts its
-        // atomics.
-        float* const dst = dq + (rowbase + qs + 16 * qt + 4 * (lane >> 4)) * M + 16 * ct + (lane & 15);
-        if (qs + QT <= N) {  // uniform
+        // Always issued (a fixed count per step: the stage waits count on
+        // it); rows past N add 0 to the row one step back, each its own (one
+        // straight sequence: a branch for whole steps measured 5 % slower).
 #pragma unroll
-          for (int r = 0; r < 4; ++r) unsafeAtomicAdd(dst + r * M, a[r]);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const bool ok = qs + 16 * qt + 4 * (lane >> 4) + r < N;
-            if (ok || N >= QT) unsafeAtomicAdd(dst + (ok ? r : r - QT) * M, ok ? a[r] : 0.f);
-          }
+        for (int r = 0; r < 4; ++r) {
+          const int qq = qs + 16 * qt + 4 * (lane >> 4) + r;
+          unsafeAtomicAdd(dq + (rowbase + (qq < N ? qq : max(qq - QT, 0))) * M + 16 * ct + (lane & 15),
+                          qq < N ? a[r] : 0.f);
         }
       }
     }
