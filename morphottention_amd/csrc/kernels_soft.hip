@@ -531,12 +531,262 @@ __global__ __launch_bounds__(256) void soft_fwd_fast_kernel(const f16* __restric
   if (__builtin_amdgcn_ballot_w64(low) != 0 && lane == 0) atomicOr(st.flag, 1);
 }
 
+// V^T-style chunk swizzle of a [row][64 keys] tile (as in attn_fwd.h)
+__device__ __forceinline__ int fswz(int r) { return (r ^ (r >> 3)) & 7; }
+// two fp32 as bf16 hi and lo pairs (hi + lo to ~2^-16 relative)
+__device__ __forceinline__ void split_bf16x2(float x0, float x1, unsigned& hi, unsigned& lo) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  asm("" : "+v"(x0), "+v"(x1));
+  hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
+  const float h0 = __builtin_bit_cast(float, hi << 16), h1 = __builtin_bit_cast(float, hi & 0xffff0000u);
+  lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0 - h0, x1 - h1}), bf16x2));
+}
+
+template <int M, int DV>
+struct FastTileCfg {
+  static constexpr int CW = 2 * M + 8;
+  static constexpr int NCH = M / 8;
+  static constexpr int WAVES = 4, QW = 32 * WAVES, KT = 64;
+  static constexpr int KCH = CW / 8, FCH = DV / 8;         // 1 KiB chunks: key rows, F^T hi (and as many lo)
+  static constexpr int NKW = (KCH + WAVES - 1) / WAVES;    // per wave (padding slots repeat the last chunk)
+  static constexpr int NFW = 2 * FCH / WAVES;
+  static_assert(2 * FCH % WAVES == 0, "F chunks must split evenly");
+  static constexpr int NPW = NKW + NFW;
+  static constexpr int FOFF = NKW * WAVES * 512, FLOFF = FOFF + FCH * 512;  // halves
+  static constexpr int STAGE = WAVES * NPW * 512;
+  static constexpr int WG_PER_CU = 2 * STAGE * 2 <= 51 * 1024 ? 3 : 2;
+  static constexpr int NSTAGE = 3 * STAGE * 2 <= (WG_PER_CU == 3 ? 51 : 78) * 1024 ? 3 : 2;
+  static constexpr int CB = DV / 32;
+};
+
+// Forward, product form, on 64-key tiles that arrive by LDS DMA (dv <= 64). As
+// soft_fwd_fast_kernel, with the key rows and both parts of F^T in stages
+// filled one tile ahead (one barrier and one row-maximum update per 64 keys
+// instead of a barrier per 32 and key rows read from memory by every wave).
+// The sign of the aggregation is folded into the query operand, so the
+// accumulator is acc = sgn log2e s, the row maximum is taken of acc itself and
+// E = 2^(acc / tau - A_i) is one fma and one exp2 per score. Bound by VALU and
+// MFMA issue together (per 32 x 32 block 16 MFMAs and about 90 VALU
+// instructions, 16 of them exp2). us, 32-key kernel -> this one: B4 N4096 H16 m16
+// dv64 causal 322 -> 268, B2 N1001 H8 m32 dv64 49.5 -> 29.1, B2 N4000 H6 m64
+// dv64 280 -> 170, m32 dv32 154 -> 111. Two stages of 128-wide values would
+// leave one workgroup per CU: there the 32-key kernel stays.
+template <int M, int DV, bool MD>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(FastTileCfg<M, DV>::WG_PER_CU, FastTileCfg<M, DV>::WG_PER_CU))) void
+soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, const float4* __restrict__ tstat,
+                     const float* __restrict__ tau_p, SoftState st, f16* __restrict__ out, float* __restrict__ zb,
+                     int N, int NP, int H, int D, int BH, int causal, float sgn) {
+  using C = FastTileCfg<M, DV>;
+  __shared__ __align__(16) f16 smem[C::NSTAGE * C::STAGE];
+  __shared__ float sbc[DV];
+  const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nqb = (N + C::QW - 1) / C::QW;
+  int bh, blk;
+  if (!(causal ? xcd_map_lpt(nqb, BH, bh, blk) : xcd_map(nqb, BH, bh, blk))) return;
+  const int qblk = causal ? nqb - 1 - blk : blk;
+  const int q0 = qblk * C::QW, qw0 = q0 + 32 * w;
+  const int b = bh / H, h = bh - b * H;
+  const int64_t rowbase = (int64_t)bh * N, fbase = (int64_t)bh * DV * NP;
+  const float tau = *tau_p;
+  const float ks = 1.f / tau, kw = sgn * kLog2e / tau;
+  for (int c = tid; c < DV; c += 256) sbc[c] = kw * (kw > 0.f ? st.vmax[bh * DV + c] : st.vmin[bh * DV + c]);
+
+  // ---- DMA: per-lane byte offsets of this wave's chunks, computed once
+  const f16* const fth = reinterpret_cast<const f16*>(st.fth) + fbase;
+  const f16* const ftl = reinterpret_cast<const f16*>(st.ftl) + fbase;
+  const unsigned sbase = (unsigned)(uintptr_t)(__attribute__((address_space(3))) f16*)smem;
+  unsigned koff[C::NKW], foff[C::NFW];
+#pragma unroll
+  for (int i = 0; i < C::NKW; ++i) {
+    const int p = 64 * min(w + C::WAVES * i, C::KCH - 1) + lane;
+    const int row = p / (C::CW / 8), col = 8 * (p % (C::CW / 8));
+    koff[i] = (unsigned)((((row & ~31) | swap23(row & 31)) * C::CW + col) * 2);
+  }
+#pragma unroll
+  for (int j = 0; j < C::NFW; ++j) {
+    const int v = (w + C::WAVES * j) % C::FCH, r = 8 * v + (lane >> 3);
+    foff[j] = (unsigned)(((int64_t)r * NP + 8 * ((lane & 7) ^ fswz(r))) * 2);
+  }
+  auto issue = [&](int t) {
+    const unsigned dst = sbase + 2u * (unsigned)((t % C::NSTAGE) * C::STAGE);
+    const int k0 = t * C::KT;
+    if (k0 + C::KT <= N) {  // uniform: no key row past N
+      const f16* kbase = ka + (rowbase + k0) * C::CW;
+#pragma unroll
+      for (int i = 0; i < C::NKW; ++i) lds_dma16_so(kbase, koff[i], dst + 1024u * (unsigned)(w + C::WAVES * i));
+    } else {  // rows past N read the last row; every score they feed is masked
+#pragma unroll
+      for (int i = 0; i < C::NKW; ++i) {
+        const int p = 64 * min(w + C::WAVES * i, C::KCH - 1) + lane;
+        const int row = p / (C::CW / 8), col = 8 * (p % (C::CW / 8));
+        const int key = min(k0 + ((row & ~31) | swap23(row & 31)), N - 1);
+        lds_dma16(ka + (rowbase + key) * C::CW + col, dst + 1024u * (unsigned)(w + C::WAVES * i));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < C::NFW; ++j) {  // zero from N to NP >= k0 + KT
+      const int v = w + C::WAVES * j;
+      lds_dma16_so((v < C::FCH ? fth : ftl) + k0, foff[j], dst + 2u * C::FOFF + 1024u * (unsigned)v);
+    }
+  };
+
+  const int q = qw0 + l32;
+  const int kend = causal ? min(N, q0 + C::QW) : N;
+  const int nkt = (kend + C::KT - 1) / C::KT;
+  issue(0);
+  if (nkt > 1) issue(1);
+  f16x8 qf[C::NCH];
+  f16x4 qaug = {};
+#pragma unroll
+  for (int c = 0; c < C::NCH; ++c) qf[c] = f16x8{};
+  if (q < N) load_query_operand<M>(qa + (rowbase + q) * C::CW, tstat[rowbase + q].x, h32, qf, qaug);
+  if (sgn < 0.f) {  // uniform
+#pragma unroll
+    for (int c = 0; c < C::NCH; ++c) qf[c] = -qf[c];
+    qaug = -qaug;
+  }
+  f32x16 o[C::CB];
+#pragma unroll
+  for (int i = 0; i < C::CB; ++i) o[i] = f32x16{};
+  // running maximum of acc over this query's keys so far, and A_i = mrow / tau
+  // as rounded once: every E and the result use this one value
+  float mrow = kNegInf, arow = kNegInf;
+  // loaded under a condition: wait on every path, or the compiler waits inside
+  // the loop, draining the DMA there
+  wait_vmcnt<0>();
+
+  // F^T fragment offsets within a stage: see attn_fwd.h
+  int fofs[2][2];
+  {
+    const int z = fswz(l32);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        fofs[x][p] = C::FOFF + l32 * C::KT + 8 * (4 * (x ^ (z >> 2)) + 2 * (p ^ ((z >> 1) & 1)) + (h32 ^ (z & 1)));
+  }
+  auto score = [&](const f16* tile, int kb) {
+    f16x8 kf[C::NCH];
+    const f16* krow = tile + (32 * kb + l32) * C::CW;
+#pragma unroll
+    for (int c = 0; c < C::NCH; ++c) kf[c] = *reinterpret_cast<const f16x8*>(krow + chunk_off<M>(c) + 8 * h32);
+    const f16x4 kx = *reinterpret_cast<const f16x4*>(krow + M + 4 * h32);
+    return mfma8(kx, qaug, code_dot<M, true>(kf, qf, f32x16{}));
+  };
+  // E of block kb (hi / lo B operands) and O^T += F^T E in three products
+  auto accumulate = [&](const f16* tile, int kb, const f32x16& acc, float nref) {
+    unsigned eh[8], el[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      split_bf16x2(fast_exp2(__builtin_fmaf(ks, acc[2 * r], nref)), fast_exp2(__builtin_fmaf(ks, acc[2 * r + 1], nref)),
+                   eh[r], el[r]);
+#pragma unroll
+    for (int part = 0; part < 2; ++part) {
+      const bf16x8 ph = __builtin_bit_cast(bf16x8, make_uint4(eh[4 * part], eh[4 * part + 1], eh[4 * part + 2], eh[4 * part + 3]));
+      const bf16x8 pl = __builtin_bit_cast(bf16x8, make_uint4(el[4 * part], el[4 * part + 1], el[4 * part + 2], el[4 * part + 3]));
+      bf16x8 fh[C::CB], fl[C::CB];
+#pragma unroll
+      for (int cb = 0; cb < C::CB; ++cb) {
+        const f16* at = tile + fofs[kb ^ (cb & 1)][part] + 32 * C::KT * cb;
+        fh[cb] = *reinterpret_cast<const bf16x8*>(at);
+        fl[cb] = *reinterpret_cast<const bf16x8*>(at + (C::FLOFF - C::FOFF));
+      }
+#pragma unroll
+      for (int cb = 0; cb < C::CB; ++cb) o[cb] = mfma_bf16(fh[cb], ph, o[cb]);
+#pragma unroll
+      for (int cb = 0; cb < C::CB; ++cb) o[cb] = mfma_bf16(fh[cb], pl, o[cb]);
+#pragma unroll
+      for (int cb = 0; cb < C::CB; ++cb) o[cb] = mfma_bf16(fl[cb], ph, o[cb]);
+    }
+  };
+
+  for (int t = 0; t < nkt; ++t) {
+    // tile t has landed in every wave's share (tile t + 1 may be in flight)
+    if (t + 1 < nkt && (t == 0 || C::NSTAGE == 3))
+      wait_vmcnt<C::NPW>();
+    else
+      wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    const int ti = t == 0 ? (C::NSTAGE == 3 ? 2 : nkt) : t + C::NSTAGE - 1;  // tiles 0 and 1 were sent before
+    if (ti < nkt) issue(ti);
+    const f16* tile = smem + (t % C::NSTAGE) * C::STAGE;
+    const int k0 = t * C::KT;
+    if (causal && k0 > qw0 + 31) continue;  // uniform: nothing unmasked for this wave
+    f32x16 a0 = score(tile, 0), a1 = score(tile, 1);
+    if ((k0 + 64 > N) || (causal && k0 + 63 > qw0) || (MD && k0 <= qw0 + 31 && k0 + 63 >= qw0)) {  // uniform
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + (r < 8 ? 8 * h32 + r : 8 + 8 * h32 + r);
+        a0[r] = (key >= N) | (causal != 0 && key > q) | (MD && key == q) ? kNegInf : a0[r];
+        a1[r] = (key + 32 >= N) | (causal != 0 && key + 32 > q) | (MD && key + 32 == q) ? kNegInf : a1[r];
+      }
+    }
+    float tm = fmaxf(a0[0], a1[0]);
+#pragma unroll
+    for (int r = 1; r < 16; ++r) tm = fmaxf(fmaxf(tm, a0[r]), a1[r]);
+    tm = fmaxf(tm, __shfl_xor(tm, 32));
+    if (__builtin_amdgcn_ballot_w64(tm > mrow) != 0) {  // some query's maximum grew: rescale its sums
+      mrow = fmaxf(mrow, tm);
+      const float an = ks * mrow;
+      const float sc = an > kNegInf ? fast_exp2(arow - an) : 1.f;
+#pragma unroll
+      for (int i = 0; i < C::CB; ++i) o[i] *= sc;
+      arow = an;
+    }
+    const float nref = arow > kNegInf ? -arow : 0.f;  // no key yet: every E is 0
+    accumulate(tile, 0, a0, nref);
+    accumulate(tile, 1, a1, nref);
+  }
+
+  // zb = A_i + B_c + log2 S_ic; out = sgn tau ln2 zb
+  __syncthreads();  // sbc (also with no tile at all)
+  bool low = false;
+  if (q < N) {
+    const float ko = sgn * tau * kLn2;
+    f16* orow = out + ((int64_t)b * N + q) * D + h * DV;
+    float* zrow = zb + (rowbase + q) * DV;
+#pragma unroll
+    for (int cb = 0; cb < C::CB; ++cb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float4 z4;
+        f16x4 o4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = 32 * cb + 8 * g + 4 * h32 + e;
+          const float sv = o[cb][4 * g + e];
+          float z = -kFltMax;
+          if (mrow > kNegInf) {
+            low = low || !(sv >= kProductFloor);
+            z = arow + sbc[c] + fast_log2(sv);
+          }
+          (&z4.x)[e] = z;
+          o4[e] = (f16)(mrow > kNegInf ? ko * z : 0.f);
+        }
+        *reinterpret_cast<float4*>(zrow + 32 * cb + 8 * g + 4 * h32) = z4;
+        *reinterpret_cast<f16x4*>(orow + 32 * cb + 8 * g + 4 * h32) = o4;
+      }
+    if (h32 == 0) st.arow[rowbase + q] = arow;
+  }
+  if (__builtin_amdgcn_ballot_w64(low) != 0 && lane == 0) atomicOr(st.flag, 1);
+}
+
 template <int M, int DV>
 static hipError_t launch_soft_fwd_fast_t(const Dims& d, const ProjBuffers& p, const float* tau, int sgn,
                                          const SoftState& st, f16* out, float* zb, hipStream_t s) {
   using C = FastCfg<M, DV>;
   const dim3 grid(xcd_grid((d.N + C::QW - 1) / C::QW, d.B * d.H));
-  if (d.mask_diag)
+  if constexpr (DV <= 64) {
+    if (d.mask_diag)
+      MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, true>), grid, dim3(256), 0, s, p.qa, p.ka, p.tstat, tau, st, out, zb,
+                     d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
+    else
+      MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, false>), grid, dim3(256), 0, s, p.qa, p.ka, p.tstat, tau, st, out,
+                     zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
+  } else if (d.mask_diag)
     MORPHO_KLAUNCH((soft_fwd_fast_kernel<M, DV, true>), grid, dim3(256), 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat,
                        tau, st, out, zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
   else

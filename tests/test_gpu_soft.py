@@ -132,6 +132,19 @@ def test_soft_ragged_lengths(N):
     _check(f"N {N}", out, zb, grads, x, params, 0.7, H, m, 0.9, False, -1, dout)
 
 
+@pytest.mark.parametrize("N,m,dv,causal,sgn", [
+    (63, 16, 32, False, 1), (64, 16, 64, True, -1), (65, 32, 64, False, -1),   # one tile, and one key of a second
+    (128, 64, 64, True, 1), (129, 64, 32, True, -1), (193, 32, 32, True, 1),   # both stage counts, masked tails
+    (400, 64, 64, False, -1), (333, 16, 32, False, 1)])
+def test_soft_forward_tiles(N, m, dv, causal, sgn):
+    """The 64-key tiles of the product-form forward (dv <= 64) at their edges."""
+    B, H = 2, 3
+    _say(f"[case] soft tiles N={N} m={m} dv={dv} causal={causal} sgn={sgn}")
+    x, params, dout = _inputs(B, N, H, m, dv, seed=7000 + N)
+    out, zb, grads = _run(x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
+    _check(f"soft tiles N={N}", out, zb, grads, x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
+
+
 def test_soft_variants_masked_diagonal_and_projection():
     """Causal with the diagonal masked leaves query 0 without keys: out 0,
     zb -FLT_MAX, and no NaN in any gradient; HardTanh01 projection."""
