@@ -1154,9 +1154,13 @@ hipError_t launch_soft_bwd(const Dims& d, const ProjBuffers& p, const f16* grad_
   MORPHO_MDV_DISPATCH(launch_soft_bwd_t, d, p, grad_out, zb, tau, sgn, g, part, run_flag, s);
 }
 
-// two waves per SIMD where the registers allow it without spilling
+// Waves per SIMD (two: at most 256 VGPRs): two where the registers allow it
+// without spilling. At one, soft_bwd_fast took 331 us at B4 N2048 H16 m32 dv64
+// causal against 234 at two (no spills either way), 248 against 177 at m32
+// dv32; at m = 64 and dv = 128 two would spill 28 to 146 values (B2 N4000 H6 m64
+// dv64 670 -> 759, dv128 866 -> 1651).
 template <int M, int DV>
-constexpr int soft_fast_bwd_waves() { return (M == 16 && DV <= 64) ? 2 : 1; }
+constexpr int soft_fast_bwd_waves() { return (M <= 32 && DV <= 64) ? 2 : 1; }
 
 // Backward, product form. With G_ic = dO_ic 2^(A_i + B_c - zb_ic) = dO_ic / S_ic:
 //     ds_ij = E_ij sum_c G_ic F_jc          (X = G F^T, then times E)
