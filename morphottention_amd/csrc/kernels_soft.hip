@@ -1154,13 +1154,24 @@ hipError_t launch_soft_bwd(const Dims& d, const ProjBuffers& p, const f16* grad_
   MORPHO_MDV_DISPATCH(launch_soft_bwd_t, d, p, grad_out, zb, tau, sgn, g, part, run_flag, s);
 }
 
-// Waves per SIMD (two: at most 256 VGPRs): two where the registers allow it
-// without spilling. At one, soft_bwd_fast took 331 us at B4 N2048 H16 m32 dv64
-// causal against 234 at two (no spills either way), 248 against 177 at m32
-// dv32; at m = 64 and dv = 128 two would spill 28 to 146 values (B2 N4000 H6 m64
-// dv64 670 -> 759, dv128 866 -> 1651).
+// Chunk swizzle of a phi tile's rows of RB bytes (as rswz in kernels_attn.hip):
+// the transposing 16 x 16 x 32 reads touch rows {r..r+3, r+8..r+11} x 2 chunks.
+template <int RB>
+__device__ __forceinline__ int pkswz(int r) {
+  static_assert(RB == 32 || RB == 64 || RB == 128, "phi row bytes");
+  if constexpr (RB == 32) return 0;
+  else if constexpr (RB == 64) return (r >> 2) & 3;
+  else return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+}
+
+// Waves per SIMD (two: at most 256 VGPRs): two for values up to 64 wide.
+// soft_bwd_fast in us, one wave -> two: B4 N2048 H16 causal m32 dv64 331 -> 234,
+// m32 dv32 248 -> 177, m64 dv64 420 -> 295, m64 dv32 348 -> 256, B2 N4000 H6 m64
+// dv64 717 -> 500 (m = 64 with the phi operand in LDS and dcb off the MFMA, 10
+// values spilled at dv 64; before that, two waves spilled 54 and took 759). At
+// dv = 128 two would spill 50 to 146 values (B2 N4000 H6 m64 866 -> 1651).
 template <int M, int DV>
-constexpr int soft_fast_bwd_waves() { return (M <= 32 && DV <= 64) ? 2 : 1; }
+constexpr int soft_fast_bwd_waves() { return DV <= 64 ? 2 : 1; }
 
 // Backward, product form. With G_ic = dO_ic 2^(A_i + B_c - zb_ic) = dO_ic / S_ic:
 //     ds_ij = E_ij sum_c G_ic F_jc          (X = G F^T, then times E)
@@ -1195,7 +1206,13 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
     int BH, int causal, float sgn) {
   constexpr int CW = 2 * M + 8, NCH = M / 8, CB = DV / 32, KW = 128, QT = 32;
   constexpr int GS = DV + 8;            // bf16 row stride of the G tiles
-  constexpr int MB = (M + 32) / 32;     // 32-code blocks of [phi | 1]
+  // dcb from the ones column where it shares a 32-code block with codes (m =
+  // 16), else from VALU sums of the same fp16 ds (a block of its own would cost
+  // 16 VGPRs and two MFMAs)
+  constexpr bool DCB_VALU = M % 32 == 0;
+  constexpr int MB = DCB_VALU ? M / 32 : M / 32 + 1;  // 32-code blocks of [phi | 1]
+  constexpr bool PHIREG = M <= 32;      // the dq product's phi operand in registers, else in LDS
+  constexpr int PRB = 2 * M;            // its LDS rows (one key's phi_hi)
   constexpr int SRB = 2 * QT;           // dS^T row bytes (one key's ds over the step's queries)
   constexpr int DQTILES = (QT / 16) * (M / 16);  // 16 x 16 dq tiles of a step
   constexpr int DQT = DQTILES >= 4 ? DQTILES / 4 : 1;  // per wave (m = 16: waves 0, 1 only)
@@ -1215,6 +1232,7 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
   constexpr int STG = OAB + 256;                    // stage bytes
   __shared__ __align__(16) char stg[2 * STG];
   __shared__ __align__(16) char sdt[KW * SRB];  // dS^T of the step: row = key, chunks swizzled by sswz
+  __shared__ __align__(16) char sPk[PHIREG ? 16 : KW * PRB];  // phi_hi of the workgroup's keys
   __shared__ float sbc[DV];
   __shared__ float red[2][4];
 
@@ -1263,11 +1281,12 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
   // and the lane offsets of the transposing A-operand reads of the dS^T tile
   // (16 x 16 x 32 layout: query 16 qt + lane % 16, keys 8 (lane / 16) + j).
   const bool dq_wave = w < DQTILES;  // uniform
-  f16x8 phib[DQT][KW / 32];
+  f16x8 phib[PHIREG ? DQT : 1][PHIREG ? KW / 32 : 1];
   int d_s[DQT][2];
 #pragma unroll
   for (int t = 0; t < DQT; ++t) {
     const int tile = w + 4 * t, qt = tile % (QT / 16), ct = tile / (QT / 16);
+    if constexpr (PHIREG)
 #pragma unroll
     for (int kc = 0; kc < KW / 32; ++kc)
 #pragma unroll
@@ -1281,6 +1300,13 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
       d_s[t][hh] = row * SRB + 16 * ((col >> 3) ^ sswz<SRB>(row)) + 2 * (col & 7);
     }
   }
+  if constexpr (!PHIREG)  // published by the first step's barriers
+    for (int v = tid; v < KW * (M / 8); v += 256) {
+      const int r = v / (M / 8), c = v % (M / 8);
+      f16x8 x = {};
+      if (k0 + r < N) x = *reinterpret_cast<const f16x8*>(qa + (rowbase + k0 + r) * CW + 8 * c);
+      *reinterpret_cast<f16x8*>(sPk + r * PRB + 16 * (c ^ pkswz<PRB>(r))) = x;
+    }
   const int kr = 32 * w + l32, sz = sswz<SRB>(kr);  // this lane's dS^T row (its key)
   if (kvalid) load_key_operand<M>(ka + (rowbase + key) * CW, h32, kf, kaug);
   f32x16 dva[CB], dka[MB];
@@ -1288,7 +1314,7 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
   for (int i = 0; i < CB; ++i) dva[i] = f32x16{};
 #pragma unroll
   for (int i = 0; i < MB; ++i) dka[i] = f32x16{};
-  float sacc = 0.f;
+  float sacc = 0.f, dcb_acc = 0.f;
 
   // DMA of the tiles of the step at query qs into stage par: wave w issues
   // pieces w, w + 4, ... of the stage, and wave 3 the A / b piece.
@@ -1420,6 +1446,14 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
     // the dS^T copy): a conversion of the product selected twice could differ
     // at fp16 ties
     asm("" : "+v"(dsh[0]), "+v"(dsh[1]));
+    if constexpr (DCB_VALU) {
+      const f16x2 ones2 = {(f16)1.f, (f16)1.f};
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          dcb_acc = __builtin_amdgcn_fdot2(f16x2{dsh[c][2 * e], dsh[c][2 * e + 1]}, ones2, dcb_acc, false);
+    }
     // dS^T row of this key: queries 8 h32 + 0..7 and 16 + 8 h32 + 0..7 are
     // logical chunks h32 and 2 + h32
 #pragma unroll
@@ -1441,8 +1475,17 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
           const char* base = sdt + 32 * kc * SRB;
           const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base + d_s[t][0]));
           const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base + d_s[t][1]));
-          a = mfma16x16(__builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)),
-                        phib[t][kc], a);
+          f16x8 phi_op;
+          if constexpr (PHIREG) {
+            phi_op = phib[t][kc];
+          } else {
+            const int row = 32 * kc + 8 * (lane >> 4) + ((lane & 15) >> 2), col = 16 * ct + 4 * (lane & 3);
+            auto at = [&](int r) { return sPk + r * PRB + 16 * ((col >> 3) ^ pkswz<PRB>(r)) + 2 * (col & 7); };
+            const s16x4 plo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at(row)));
+            const s16x4 phi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at(row + 4)));
+            phi_op = __builtin_bit_cast(f16x8, __builtin_shufflevector(plo, phi, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+          a = mfma16x16(__builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)), phi_op, a);
         }
         // rows: queries 16 qt + 4 (lane / 16) + r; column: code 16 ct + lane % 16.
         // Always issued (a fixed count per step: the stage waits count on
@@ -1460,7 +1503,9 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
 
   // ---- epilogue: dV_jc = F_jc (G^T E)_cj; dk, dcb; sum dV * w for dtau
   float sv = 0.f;
+  const float dcb_sum = dcb_acc + __shfl_xor(dcb_acc, 32);  // lanes l, l + 32: the same key
   if (kvalid) {
+    if (DCB_VALU && h32 == 0) dcb[rowbase + key] += dcb_sum;  // the prep wrote the row sum
     f16* drow = dzv + (tokbase + key) * (int64_t)(HM + D) + HM + h * DV;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
@@ -1483,7 +1528,7 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
       for (int r = 0; r < 16; ++r) {
         const int code = 32 * mb + acc_row(r, lane);
         if (code < M) dk[(rowbase + key) * M + code] = dka[mb][r];
-        if (code == M) dcb[rowbase + key] += dka[mb][r];  // the prep wrote the row sum
+        if (!DCB_VALU && code == M) dcb[rowbase + key] += dka[mb][r];
       }
   }
 #pragma unroll
