@@ -1196,8 +1196,11 @@ constexpr int soft_fast_bwd_waves() { return DV <= 64 ? 2 : 1; }
 // per term, against the 1e-2 bar. (Three MFMAs of hi/lo pairs each had been
 // used here; the products of G, E and F keep their bf16 hi/lo pairs, whose
 // range they need.)
-template <int M, int DV, bool MD>
-__global__ __launch_bounds__(256)
+// SPLIT: two groups of four waves per 128 keys, taking the query steps in turn
+// through stages and dS^T tiles of their own; the second group's sums are added
+// to the first's at the end.
+template <int M, int DV, bool MD, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 512 : 256)
 __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_waves<M, DV>()))) void soft_bwd_fast_kernel(
     const f16* __restrict__ qa, const f16* __restrict__ ka, const f16* __restrict__ vt,
     const uint8_t* __restrict__ vlo, const float4* __restrict__ tstat, const float* __restrict__ tau_p, SoftState st,
@@ -1230,14 +1233,17 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
   constexpr int NPC = NQP + 2 * NGP;
   constexpr int OGH = NQP * 1024, OGL = OGH + NGP * 1024, OAB = OGL + NGP * 1024;
   constexpr int STG = OAB + 256;                    // stage bytes
-  __shared__ __align__(16) char stg[2 * STG];
-  __shared__ __align__(16) char sdt[KW * SRB];  // dS^T of the step: row = key, chunks swizzled by sswz
+  constexpr int NG = SPLIT ? 2 : 1;                 // groups of four waves
+  __shared__ __align__(16) char stg_[NG * 2 * STG];
+  __shared__ __align__(16) char sdt_[NG * KW * SRB];  // dS^T of the step: row = key, chunks swizzled by sswz
   __shared__ __align__(16) char sPk[PHIREG ? 16 : KW * PRB];  // phi_hi of the workgroup's keys
   __shared__ float sbc[DV];
-  __shared__ float red[2][4];
+  __shared__ float red[2][4 * NG];
 
   const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv % 4, grp = wv / 4;  // wave of the group, group
+  char* const stg = stg_ + (NG == 1 ? 0 : grp * (2 * STG));
+  char* const sdt = sdt_ + (NG == 1 ? 0 : grp * (KW * SRB));
   const int nkb = (N + KW - 1) / KW;
   int bh, kblk;
   if (*st.flag != 0 || !(causal ? xcd_map_lpt(nkb, BH, bh, kblk) : xcd_map(nkb, BH, bh, kblk))) {
@@ -1301,7 +1307,7 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
     }
   }
   if constexpr (!PHIREG)  // published by the first step's barriers
-    for (int v = tid; v < KW * (M / 8); v += 256) {
+    for (int v = tid; v < KW * (M / 8); v += 256 * NG) {
       const int r = v / (M / 8), c = v % (M / 8);
       f16x8 x = {};
       if (k0 + r < N) x = *reinterpret_cast<const f16x8*>(qa + (rowbase + k0 + r) * CW + 8 * c);
@@ -1345,20 +1351,28 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
   wait_vmcnt<0>();
 
   const int qstart = causal ? k0 : 0;
-  if (qstart < N) issue(qstart, 0);
+  // the group's steps start at qs0 and advance by NG steps; every group takes
+  // part in the barriers of the longest
+  const int qs0 = qstart + (NG == 1 ? 0 : grp * QT);
+  if (qs0 < N) issue(qs0, 0);
   int par = 0;
-  for (int qs = qstart; qs < N; qs += QT, par ^= 1) {
+  for (int qs = qs0; NG == 1 ? qs < N : qs - grp * QT < N; qs += NG * QT, par ^= 1) {
+    if (NG == 2 && qs >= N) {  // uniform over the group: the other group's last step
+      __syncthreads();
+      __syncthreads();
+      continue;
+    }
     // this step's stage has landed (the previous step's dq atomics, issued
     // after it, may still be in flight), for every wave after the barrier,
     // which also frees the other stage and the dS^T tile
-    if (qs == qstart)
+    if (qs == qs0)
       wait_vmcnt_lgkm0<0>();
     else if (dq_wave)  // uniform
       wait_vmcnt_lgkm0<4 * DQT>();
     else
       wait_vmcnt_lgkm0<0>();
     __syncthreads();
-    if (qs + QT < N) issue(qs + QT, par ^ 1);
+    if (qs + NG * QT < N) issue(qs + NG * QT, par ^ 1);
     const char* sq = stg + par * STG;
     const bf16* sgh = reinterpret_cast<const bf16*>(sq + OGH);
     const bf16* sgl = reinterpret_cast<const bf16*>(sq + OGL);
@@ -1503,8 +1517,44 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
 
   // ---- epilogue: dV_jc = F_jc (G^T E)_cj; dk, dcb; sum dV * w for dtau
   float sv = 0.f;
+  if constexpr (NG == 2) {
+    constexpr int RS = 256;  // floats per register handed over
+    static_assert(RS * 16 * CB * 4 <= NG * 2 * STG && RS * (16 * MB + 1) * 4 <= NG * 2 * STG,
+                  "partial sums must fit the stages");
+    float* ex = reinterpret_cast<float*>(stg_) + (tid & 255);
+    __syncthreads();  // every wave is done with the stages
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < CB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[RS * (16 * i + r)] = dva[i][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < CB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dva[i][r] += ex[RS * (16 * i + r)];
+    }
+    __syncthreads();
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[RS * (16 * i + r)] = dka[i][r];
+      ex[RS * 16 * MB] = dcb_acc;
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dka[i][r] += ex[RS * (16 * i + r)];
+      dcb_acc += ex[RS * 16 * MB];
+    }
+  }
   const float dcb_sum = dcb_acc + __shfl_xor(dcb_acc, 32);  // lanes l, l + 32: the same key
-  if (kvalid) {
+  if (kvalid && (NG == 1 || grp == 0)) {
     if (DCB_VALU && h32 == 0) dcb[rowbase + key] += dcb_sum;  // the prep wrote the row sum
     f16* drow = dzv + (tokbase + key) * (int64_t)(HM + D) + HM + h * DV;
 #pragma unroll
@@ -1537,12 +1587,14 @@ __attribute__((amdgpu_waves_per_eu(soft_fast_bwd_waves<M, DV>(), soft_fast_bwd_w
     sv += __shfl_xor(sv, sh);
   }
   if (lane == 0) {
-    red[0][w] = sacc;
-    red[1][w] = sv;
+    red[0][wv] = sacc;
+    red[1][wv] = sv;
   }
   __syncthreads();
   if (tid == 0) {
-    part[2 * blockIdx.x] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    float a = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    if constexpr (NG == 2) a += (red[0][4] + red[0][5]) + (red[0][6] + red[0][7]);
+    part[2 * blockIdx.x] = a;
     part[2 * blockIdx.x + 1] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
   }
 }
@@ -1556,14 +1608,30 @@ static hipError_t launch_soft_bwd_fast_t(const Dims& d, const ProjBuffers& p, co
   const dim3 grid(xcd_grid((d.N + 127) / 128, d.B * d.H));
   const auto* h = reinterpret_cast<const bf16*>(gh);
   const auto* l = reinterpret_cast<const bf16*>(gl);
+#define MORPHO_SOFT_BWD(MD_, SPLIT_)                                                                                 \
+  MORPHO_KLAUNCH((soft_bwd_fast_kernel<M, DV, MD_, SPLIT_>), grid, dim3(SPLIT_ ? 512 : 256), 0, s, p.qa, p.ka, p.vt, \
+                 p.vlo, p.tstat, tau, st, h, l, g.dq, g.dk, g.dcb, g.dzv, part, d.N, d.NP, d.H, d.D, d.HM,           \
+                 d.B * d.H, d.causal, (float)sgn)
+  // as the softmax backward: the split shape where one workgroup's chain of
+  // steps is at least the mean work of a CU. soft_bwd_fast in us, regular ->
+  // split: B2 N1001 H8 m16 dv64 74 -> 55, m32 83 -> 60, m64 116 -> 77, B1 H16
+  // causal N3000 m16 170 -> 121, m64 272 -> 179, N4096 m32 274 -> 223; B1 N300 H2
+  // m16 32 -> 28. Two groups at dv = 128 would need more registers than two
+  // waves per SIMD have.
+  if constexpr (DV <= 64) {
+    if (d.N > 256 && few_long_chains(d, 528)) {
+      if (d.mask_diag)
+        MORPHO_SOFT_BWD(true, true);
+      else
+        MORPHO_SOFT_BWD(false, true);
+      return hipGetLastError();
+    }
+  }
   if (d.mask_diag)
-    MORPHO_KLAUNCH((soft_bwd_fast_kernel<M, DV, true>), grid, dim3(256), 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat,
-                       tau, st, h, l, g.dq, g.dk, g.dcb, g.dzv, part, d.N, d.NP, d.H, d.D, d.HM, d.B * d.H,
-                       d.causal, (float)sgn);
+    MORPHO_SOFT_BWD(true, false);
   else
-    MORPHO_KLAUNCH((soft_bwd_fast_kernel<M, DV, false>), grid, dim3(256), 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat,
-                       tau, st, h, l, g.dq, g.dk, g.dcb, g.dzv, part, d.N, d.NP, d.H, d.D, d.HM, d.B * d.H,
-                       d.causal, (float)sgn);
+    MORPHO_SOFT_BWD(false, false);
+#undef MORPHO_SOFT_BWD
   return hipGetLastError();
 }
 

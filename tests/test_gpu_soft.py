@@ -135,9 +135,11 @@ def test_soft_ragged_lengths(N):
 @pytest.mark.parametrize("N,m,dv,causal,sgn", [
     (63, 16, 32, False, 1), (64, 16, 64, True, -1), (65, 32, 64, False, -1),   # one tile, and one key of a second
     (128, 64, 64, True, 1), (129, 64, 32, True, -1), (193, 32, 32, True, 1),   # both stage counts, masked tails
-    (400, 64, 64, False, -1), (333, 16, 32, False, 1)])
+    (400, 64, 64, False, -1), (333, 16, 32, False, 1),       # with the split backward: odd numbers of steps
+    (290, 64, 32, True, 1), (385, 16, 64, True, -1), (257, 32, 64, False, 1)])
 def test_soft_forward_tiles(N, m, dv, causal, sgn):
-    """The 64-key tiles of the product-form forward (dv <= 64) at their edges."""
+    """The 64-key tiles of the product-form forward (dv <= 64) at their edges,
+    and from 257 tokens on the split shape of its backward."""
     B, H = 2, 3
     _say(f"[case] soft tiles N={N} m={m} dv={dv} causal={causal} sgn={sgn}")
     x, params, dout = _inputs(B, N, H, m, dv, seed=7000 + N)
