@@ -543,11 +543,12 @@ __device__ __forceinline__ void split_bf16x2(float x0, float x1, unsigned& hi, u
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0 - h0, x1 - h1}), bf16x2));
 }
 
-template <int M, int DV>
+// SPLIT: two groups of four waves per 128 queries, taking the key tiles in turn
+template <int M, int DV, bool SPLIT>
 struct FastTileCfg {
   static constexpr int CW = 2 * M + 8;
   static constexpr int NCH = M / 8;
-  static constexpr int WAVES = 4, QW = 32 * WAVES, KT = 64;
+  static constexpr int WAVES = 4, QW = 32 * WAVES, KT = 64, NG = SPLIT ? 2 : 1;
   static constexpr int KCH = CW / 8, FCH = DV / 8;         // 1 KiB chunks: key rows, F^T hi (and as many lo)
   static constexpr int NKW = (KCH + WAVES - 1) / WAVES;    // per wave (padding slots repeat the last chunk)
   static constexpr int NFW = 2 * FCH / WAVES;
@@ -555,8 +556,9 @@ struct FastTileCfg {
   static constexpr int NPW = NKW + NFW;
   static constexpr int FOFF = NKW * WAVES * 512, FLOFF = FOFF + FCH * 512;  // halves
   static constexpr int STAGE = WAVES * NPW * 512;
-  static constexpr int WG_PER_CU = 2 * STAGE * 2 <= 51 * 1024 ? 3 : 2;
-  static constexpr int NSTAGE = 3 * STAGE * 2 <= (WG_PER_CU == 3 ? 51 : 78) * 1024 ? 3 : 2;
+  static constexpr int WG_PER_CU = SPLIT ? 1 : 2 * STAGE * 2 <= 51 * 1024 ? 3 : 2;
+  static constexpr int WAVES_PER_EU = WG_PER_CU * NG;
+  static constexpr int NSTAGE = 3 * STAGE * 2 <= (WG_PER_CU == 3 ? 51 : 78) * 1024 ? 3 : 2;  // of a group
   static constexpr int CB = DV / 32;
 };
 
@@ -572,17 +574,21 @@ struct FastTileCfg {
 // dv64 causal 322 -> 268, B2 N1001 H8 m32 dv64 49.5 -> 29.1, B2 N4000 H6 m64
 // dv64 280 -> 170, m32 dv32 154 -> 111. Two stages of 128-wide values would
 // leave one workgroup per CU: there the 32-key kernel stays.
-template <int M, int DV, bool MD>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(FastTileCfg<M, DV>::WG_PER_CU, FastTileCfg<M, DV>::WG_PER_CU))) void
+// SPLIT: each group keeps its own running maximum; the second hands its maximum
+// and sums over at the end.
+template <int M, int DV, bool MD, bool SPLIT>
+__global__ __launch_bounds__((256 * FastTileCfg<M, DV, SPLIT>::NG))
+__attribute__((amdgpu_waves_per_eu(FastTileCfg<M, DV, SPLIT>::WAVES_PER_EU, FastTileCfg<M, DV, SPLIT>::WAVES_PER_EU))) void
 soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, const float4* __restrict__ tstat,
                      const float* __restrict__ tau_p, SoftState st, f16* __restrict__ out, float* __restrict__ zb,
                      int N, int NP, int H, int D, int BH, int causal, float sgn) {
-  using C = FastTileCfg<M, DV>;
-  __shared__ __align__(16) f16 smem[C::NSTAGE * C::STAGE];
+  using C = FastTileCfg<M, DV, SPLIT>;
+  __shared__ __align__(16) f16 smem_[C::NG * C::NSTAGE * C::STAGE];
   __shared__ float sbc[DV];
   const int tid = threadIdx.x, lane = tid & 63, h32 = lane >> 5, l32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wv % C::WAVES, grp = wv / C::WAVES;  // wave of the group, group
+  f16* const smem = smem_ + (C::NG == 1 ? 0 : grp * (C::NSTAGE * C::STAGE));
   const int nqb = (N + C::QW - 1) / C::QW;
   int bh, blk;
   if (!(causal ? xcd_map_lpt(nqb, BH, bh, blk) : xcd_map(nqb, BH, bh, blk))) return;
@@ -612,7 +618,7 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
   }
   auto issue = [&](int t) {
     const unsigned dst = sbase + 2u * (unsigned)((t % C::NSTAGE) * C::STAGE);
-    const int k0 = t * C::KT;
+    const int k0 = (C::NG == 1 ? t : 2 * t + grp) * C::KT;
     if (k0 + C::KT <= N) {  // uniform: no key row past N
       const f16* kbase = ka + (rowbase + k0) * C::CW;
 #pragma unroll
@@ -635,8 +641,10 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
 
   const int q = qw0 + l32;
   const int kend = causal ? min(N, q0 + C::QW) : N;
-  const int nkt = (kend + C::KT - 1) / C::KT;
-  issue(0);
+  // the group's own tiles: its t-th is tile NG t + grp; nit barriers for all
+  const int nall = (kend + C::KT - 1) / C::KT, nit = (nall + C::NG - 1) / C::NG;
+  const int nkt = C::NG == 1 ? nall : (nall - grp + 1) / 2;
+  if (C::NG == 1 || nkt > 0) issue(0);
   if (nkt > 1) issue(1);
   f16x8 qf[C::NCH];
   f16x4 qaug = {};
@@ -703,7 +711,7 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
     }
   };
 
-  for (int t = 0; t < nkt; ++t) {
+  for (int t = 0; t < nit; ++t) {
     // tile t has landed in every wave's share (tile t + 1 may be in flight)
     if (t + 1 < nkt && (t == 0 || C::NSTAGE == 3))
       wait_vmcnt<C::NPW>();
@@ -713,8 +721,8 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
     const int ti = t == 0 ? (C::NSTAGE == 3 ? 2 : nkt) : t + C::NSTAGE - 1;  // tiles 0 and 1 were sent before
     if (ti < nkt) issue(ti);
     const f16* tile = smem + (t % C::NSTAGE) * C::STAGE;
-    const int k0 = t * C::KT;
-    if (causal && k0 > qw0 + 31) continue;  // uniform: nothing unmasked for this wave
+    const int k0 = (C::NG == 1 ? t : 2 * t + grp) * C::KT;
+    if ((C::NG == 2 && t >= nkt) || (causal && k0 > qw0 + 31)) continue;  // uniform: nothing (unmasked) for this wave
     f32x16 a0 = score(tile, 0), a1 = score(tile, 1);
     if ((k0 + 64 > N) || (causal && k0 + 63 > qw0) || (MD && k0 <= qw0 + 31 && k0 + 63 >= qw0)) {  // uniform
 #pragma unroll
@@ -742,7 +750,31 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
   }
 
   // zb = A_i + B_c + log2 S_ic; out = sgn tau ln2 zb
-  __syncthreads();  // sbc (also with no tile at all)
+  __syncthreads();  // sbc (also with no tile at all), and every wave is done with the stages
+  if constexpr (C::NG == 2) {
+    constexpr int NR = DV / 2 + 2;  // registers to hand over
+    static_assert(256 * NR * 4 <= 2 * C::NG * C::NSTAGE * C::STAGE, "partial sums must fit the stages");
+    float* ex = reinterpret_cast<float*>(smem_) + (tid & 255);
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < C::CB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[256 * (16 * i + r)] = o[i][r];
+      ex[256 * (NR - 2)] = mrow;
+      ex[256 * (NR - 1)] = arow;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = ex[256 * (NR - 2)], a1 = ex[256 * (NR - 1)];
+    const float an = m1 > mrow ? a1 : arow;  // A_i of the larger maximum
+    const float s0 = arow > kNegInf ? fast_exp2(arow - an) : 0.f, s1 = a1 > kNegInf ? fast_exp2(a1 - an) : 0.f;
+#pragma unroll
+    for (int i = 0; i < C::CB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[i][r] = o[i][r] * s0 + ex[256 * (16 * i + r)] * s1;
+    mrow = fmaxf(mrow, m1);
+    arow = an;
+  }
   bool low = false;
   if (q < N) {
     const float ko = sgn * tau * kLn2;
@@ -780,12 +812,22 @@ static hipError_t launch_soft_fwd_fast_t(const Dims& d, const ProjBuffers& p, co
   using C = FastCfg<M, DV>;
   const dim3 grid(xcd_grid((d.N + C::QW - 1) / C::QW, d.B * d.H));
   if constexpr (DV <= 64) {
-    if (d.mask_diag)
-      MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, true>), grid, dim3(256), 0, s, p.qa, p.ka, p.tstat, tau, st, out, zb,
-                     d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
+#define MORPHO_SOFT_TILE(MD_, SPLIT_)                                                                               \
+  MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, MD_, SPLIT_>), grid, dim3(SPLIT_ ? 512 : 256), 0, s, p.qa, p.ka,      \
+                 p.tstat, tau, st, out, zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn)
+    // the split shape as in the softmax forward. soft_fwd_fast in us, one group
+    // -> two: B2 N1001 H8 m32 29.0 -> 23.6, B1 N2048 H16 m16 50 -> 42, B1 H16
+    // causal N3000 m64 91 -> 71, N4096 m32 108 -> 91, B1 N300 H2 m16 11.3 -> 10.5
+    const bool split = few_long_chains(d, 528);
+    if (d.mask_diag && split)
+      MORPHO_SOFT_TILE(true, true);
+    else if (d.mask_diag)
+      MORPHO_SOFT_TILE(true, false);
+    else if (split)
+      MORPHO_SOFT_TILE(false, true);
     else
-      MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, false>), grid, dim3(256), 0, s, p.qa, p.ka, p.tstat, tau, st, out,
-                     zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
+      MORPHO_SOFT_TILE(false, false);
+#undef MORPHO_SOFT_TILE
   } else if (d.mask_diag)
     MORPHO_KLAUNCH((soft_fwd_fast_kernel<M, DV, true>), grid, dim3(256), 0, s, p.qa, p.ka, p.vt, p.vlo, p.tstat,
                        tau, st, out, zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn);
