@@ -560,8 +560,7 @@ MORPHO_EXPORT int morpho_soft_forward(const void* X, const void* W_phi, const vo
     return MORPHO_OK;
   }
   // product form on MFMA; the element-wise kernel runs only if some output
-  // failed its check (the flag, cleared by soft_colext)
-  MORPHO_LAUNCH("soft_colext", launch_soft_colext(d, p, ss, s));
+  // failed its check (the flag, cleared by soft_fvals)
   MORPHO_LAUNCH("soft_fvals", launch_soft_fvals(d, p, tau, sgn, ss, s));
   MORPHO_LAUNCH("soft_fwd_fast", launch_soft_fwd_fast(d, p, tau, sgn, ss, o, zb, s));
   MORPHO_LAUNCH("soft_fwd", launch_soft_fwd(d, p, tau, sgn, o, zb, ss.flag, s));

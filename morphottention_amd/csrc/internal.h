@@ -175,7 +175,6 @@ struct SoftState {
 // Element-wise kernels; with run_flag they do nothing unless *run_flag != 0.
 hipError_t launch_soft_fwd(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, _Float16* out, float* zb,
                            const int* run_flag, hipStream_t s);
-hipError_t launch_soft_colext(const Dims& d, const ProjBuffers& p, const SoftState& st, hipStream_t s);
 hipError_t launch_soft_fvals(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, const SoftState& st,
                              hipStream_t s);
 hipError_t launch_soft_fwd_fast(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, const SoftState& st,

@@ -290,18 +290,28 @@ __device__ __forceinline__ void split_bf16(float x, bf16& hi, bf16& lo) {
 }
 constexpr float kProductFloor = 0x1p-80f;
 
-// Per (head, value column): max and min of V over the head's keys (the
-// column reference B_c is kw max V for kw > 0, kw min V for kw < 0). One wave
-// per column. Block 0 also clears the fallback flag of this call.
-__global__ __launch_bounds__(256) void soft_colext_kernel(const f16* __restrict__ vt, const uint8_t* __restrict__ vlo,
-                                                          float* __restrict__ vmax, float* __restrict__ vmin,
-                                                          int* __restrict__ flag, int N, int NP, int DV, int ncol) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
-  const int col = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (col >= ncol) return;
+// Per (head, value column): the maximum and minimum of V over the head's keys
+// (the column reference B_c is kw max V for kw > 0, kw min V for kw < 0), then
+// F^T = 2^(w - B_c) of its keys as bf16 hi / lo pairs, [B*H, DV, NP] with keys
+// contiguous: the tiles every query block of the product-form forward reads.
+// WPC waves per column, 8 keys per lane and pass; the second pass over V reads
+// lines that the first just brought in. Bound by HBM (3 bytes read and 4
+// written per value). As two launches: 9.0 + 20.6 us at B4 N4096 H16 dv64, 4.0 +
+// 4.4 at B2 N1001 H8 dv64; now 28.4 and 4.4. Block 0 also clears the fallback
+// flag of this call.
+template <int WPC>
+__global__ __launch_bounds__(256) void soft_fvals_kernel(const f16* __restrict__ vt, const uint8_t* __restrict__ vlo,
+                                                         const float* __restrict__ tau_p, SoftState st, int N, int NP,
+                                                         int DV, int ncol, float sgn) {
+  __shared__ float ext[2][4];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *st.flag = 0;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col = WPC == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
+  const int first = 8 * (WPC == 1 ? lane : (int)threadIdx.x), step = 512 * WPC;
+  if (col >= ncol) return;  // uniform over the column's waves
   const int bh = col / DV, c = col - bh * DV;
   float hi = kNegInf, lo = -kNegInf;
-  for (int k0 = 8 * lane; k0 < N; k0 += 512) {  // 8 keys per lane and pass
+  for (int k0 = first; k0 < N; k0 += step) {
     float v[8];
     load_values8(vt, vlo, bh, DV, NP, c, k0, v);
 #pragma unroll
@@ -316,53 +326,49 @@ __global__ __launch_bounds__(256) void soft_colext_kernel(const f16* __restrict_
     hi = fmaxf(hi, __shfl_xor(hi, sh));
     lo = fminf(lo, __shfl_xor(lo, sh));
   }
-  if (lane == 0) {
-    vmax[col] = hi;
-    vmin[col] = lo;
+  if constexpr (WPC == 4) {
+    if (lane == 0) {
+      ext[0][wv] = hi;
+      ext[1][wv] = lo;
+    }
+    __syncthreads();
+    hi = fmaxf(fmaxf(ext[0][0], ext[0][1]), fmaxf(ext[0][2], ext[0][3]));
+    lo = fminf(fminf(ext[1][0], ext[1][1]), fminf(ext[1][2], ext[1][3]));
   }
-}
-
-hipError_t launch_soft_colext(const Dims& d, const ProjBuffers& p, const SoftState& st, hipStream_t s) {
-  const int ncol = d.B * d.H * d.DV;
-  MORPHO_KLAUNCH(soft_colext_kernel, dim3((unsigned)((ncol + 3) / 4)), dim3(256), 0, s, p.vt, p.vlo, st.vmax,
-                     st.vmin, st.flag, d.N, d.NP, d.DV, ncol);
-  return hipGetLastError();
-}
-
-// F^T = 2^(w - B_c) of every (head, column, key) as bf16 hi / lo pairs,
-// [B*H, DV, NP] with keys contiguous: the tiles every query block of the
-// product-form forward reads. One thread per 8 keys of a column.
-__global__ __launch_bounds__(256) void soft_fvals_kernel(const f16* __restrict__ vt, const uint8_t* __restrict__ vlo,
-                                                         const float* __restrict__ tau_p, SoftState st, int N, int NP,
-                                                         int DV, int64_t nchunks, float sgn) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= nchunks) return;
-  const int64_t col = i / (NP / 8);  // bh * DV + c
-  const int k0 = 8 * (int)(i - col * (NP / 8));
-  const int bh = (int)(col / DV), c = (int)(col - (int64_t)bh * DV);
+  if (first == 0) {
+    st.vmax[col] = hi;
+    st.vmin[col] = lo;
+  }
   const float kw = sgn * kLog2e / *tau_p;
-  const float bc = kw * (kw > 0.f ? st.vmax[col] : st.vmin[col]);
-  bf16x8 hi, lo;
-  float v[8];
-  load_values8(vt, vlo, bh, DV, NP, c, k0, v);
+  const float bc = kw * (kw > 0.f ? hi : lo);
+  for (int k0 = first; k0 < NP; k0 += step) {
+    bf16x8 fh, fl;
+    float v[8];
+    load_values8(vt, vlo, bh, DV, NP, c, k0, v);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float ev = fast_exp2(kw * v[j] - bc);
-    const float f = k0 + j < N ? ev : 0.f;
-    bf16 h, l;
-    split_bf16(f, h, l);
-    hi[j] = h;
-    lo[j] = l;
+    for (int j = 0; j < 8; ++j) {
+      const float ev = fast_exp2(kw * v[j] - bc);
+      const float f = k0 + j < N ? ev : 0.f;
+      bf16 h, l;
+      split_bf16(f, h, l);
+      fh[j] = h;
+      fl[j] = l;
+    }
+    *reinterpret_cast<bf16x8*>(st.fth + (int64_t)col * NP + k0) = fh;
+    *reinterpret_cast<bf16x8*>(st.ftl + (int64_t)col * NP + k0) = fl;
   }
-  *reinterpret_cast<bf16x8*>(st.fth + col * NP + k0) = hi;
-  *reinterpret_cast<bf16x8*>(st.ftl + col * NP + k0) = lo;
 }
 
+// Four waves per column beyond one wave's first pass (512 keys).
 hipError_t launch_soft_fvals(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, const SoftState& st,
                              hipStream_t s) {
-  const int64_t n = (int64_t)d.B * d.H * d.DV * (d.NP / 8);
-  MORPHO_KLAUNCH(soft_fvals_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N,
-                     d.NP, d.DV, n, (float)sgn);
+  const int ncol = d.B * d.H * d.DV;
+  if (d.NP > 512)
+    MORPHO_KLAUNCH(soft_fvals_kernel<4>, dim3((unsigned)ncol), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N, d.NP, d.DV,
+                   ncol, (float)sgn);
+  else
+    MORPHO_KLAUNCH(soft_fvals_kernel<1>, dim3((unsigned)((ncol + 3) / 4)), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N,
+                   d.NP, d.DV, ncol, (float)sgn);
   return hipGetLastError();
 }
 
