@@ -271,7 +271,8 @@ def test_projection_tile_128x160(B, N, D, H, causal):
     (64, 129, 16, 64, 64),   # 256 x 256 tiles, half-tile column groups, one live token in the last group
     (52, 128, 5, 64, 64),    # heads must not straddle 160-column tiles
     (64, 199, 12, 64, 64),   # 128 x 256 tiles; backward GEMM tiles in 8 equal runs, cut inside a row panel
-], ids=["N31", "N33", "N197", "N71", "t320", "t256", "H5m64", "t128x256"])
+    (313, 128, 5, 64, 32),   # 128 x 256 tiles, natural column order, last column tile ragged
+], ids=["N31", "N33", "N197", "N71", "t320", "t256", "H5m64", "t128x256", "t128ragged"])
 def test_projection_rows_and_tiles(B, N, H, m, dv):
     """The projection's padded rows (N % 8 != 0), its tile shapes and column
     orders against the fp32 oracle."""
