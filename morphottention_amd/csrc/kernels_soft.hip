@@ -572,10 +572,11 @@ struct FastTileCfg {
 // soft_fwd_fast_kernel, with the key rows and both parts of F^T in stages
 // filled one tile ahead (one barrier and one row-maximum update per 64 keys
 // instead of a barrier per 32 and key rows read from memory by every wave).
-// The sign of the aggregation is folded into the query operand, so the
-// accumulator is acc = sgn log2e s, the row maximum is taken of acc itself and
-// E = 2^(acc / tau - A_i) is one fma and one exp2 per score. Bound by VALU and
-// MFMA issue together (per 32 x 32 block 16 MFMAs and about 90 VALU
+// The sign of sgn / tau is folded into the query operand, so that the
+// accumulator acc grows with u = acc / |tau| (also at the negative tau that a
+// learnable temperature can reach), the row maximum is taken of acc itself and
+// E = 2^(acc / |tau| - A_i) is one fma and one exp2 per score. Bound by VALU
+// and MFMA issue together (per 32 x 32 block 16 MFMAs and about 90 VALU
 // instructions, 16 of them exp2). us, 32-key kernel -> this one: B4 N4096 H16 m16
 // dv64 causal 322 -> 268, B2 N1001 H8 m32 dv64 49.5 -> 29.1, B2 N4000 H6 m64
 // dv64 280 -> 170, m32 dv32 154 -> 111. Two stages of 128-wide values would
@@ -603,7 +604,7 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
   const int b = bh / H, h = bh - b * H;
   const int64_t rowbase = (int64_t)bh * N, fbase = (int64_t)bh * DV * NP;
   const float tau = *tau_p;
-  const float ks = 1.f / tau, kw = sgn * kLog2e / tau;
+  const float ks = 1.f / fabsf(tau), kw = sgn * kLog2e / tau;
   for (int c = tid; c < DV; c += 256) sbc[c] = kw * (kw > 0.f ? st.vmax[bh * DV + c] : st.vmin[bh * DV + c]);
 
   // ---- DMA: per-lane byte offsets of this wave's chunks, computed once
@@ -657,7 +658,7 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
 #pragma unroll
   for (int c = 0; c < C::NCH; ++c) qf[c] = f16x8{};
   if (q < N) load_query_operand<M>(qa + (rowbase + q) * C::CW, tstat[rowbase + q].x, h32, qf, qaug);
-  if (sgn < 0.f) {  // uniform
+  if ((sgn < 0.f) != (tau < 0.f)) {  // uniform
 #pragma unroll
     for (int c = 0; c < C::NCH; ++c) qf[c] = -qf[c];
     qaug = -qaug;

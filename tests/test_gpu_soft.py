@@ -267,6 +267,59 @@ def test_product_form_matches_elementwise_kernels(tau, sgn, causal):
     assert do <= 0.0
 
 
+@pytest.mark.parametrize("dv", [64, 128])
+@pytest.mark.parametrize("sgn", [1, -1], ids=["dilation", "erosion"])
+@pytest.mark.parametrize("B,N", [(1, 256), (150, 256), (1, 200)], ids=["split", "one-group", "masked-tail"])
+def test_negative_temperature(B, N, sgn, dv):
+    """A learnable tau can cross zero, where the row's largest exponent is at
+    its smallest score. One token against N - 1 equal ones, with tau such that
+    their exponents are 126.5 apart: referred to the smaller one the N - 1 terms
+    would add up to +inf without any of them being infinite, and masked scores
+    would be +inf. The product form holds (its flag stays 0)."""
+    H, m = 2, 16
+    x, params, _ = _inputs(1, N, H, m, dv, seed=1200, x_mult=3.0)
+    params[3] = (0.1 * params[3]).half()                       # the columns' values stay within the product form
+    x[:, 1:] = -x[:, :1]
+    x = x.expand(B, -1, -1).contiguous()
+    _, q, k, qb, cb = mo.project(x[:1].double(), params[0].double(), torch.ones_like(params[1]).double(),
+                                 torch.ones_like(params[2]).double(), H, m)
+    params[1], params[2] = torch.ones_like(params[1]), torch.ones_like(params[2])
+    s = mo.scores(q, k, qb, cb, 1.0)[0, 0, 0]                   # head 0, query 0
+    tau = -(s[0] - s[1]).item() * math.log2(math.e) / 126.5
+    assert tau < -0.05 and s[0] > s[1]
+    t = torch.tensor([tau], dtype=torch.float32, device="cuda")
+    out, zb, ws = torch.ops.morphottention.soft_forward(x, *params, t, H, m, 1.0, False, sgn, 0)
+    flag = _flag(ws, B, N, H * dv, H, m)
+    ref, ref_zb = mo.soft_morph_ref(x[:1].float(), *(p.float() for p in params), tau, H, m, sgn=sgn, return_zb=True)
+    err = ((out.float() - ref).abs() - _half_ulp(ref)).max().item()
+    zerr = (abs(tau) * math.log(2.0) * (zb.view(B, H, N, dv) - ref_zb.view(1, H, N, dv)).abs()).max().item()
+    vmax = mo.values(x[:1].float(), params[3].float(), H).abs().max().item()
+    _say(f"[soft] negative tau {tau:.4f} B={B} N={N} sgn={sgn:+d} dv={dv}: beyond rounding {err:.2e} zb {zerr:.2e} "
+         f"flag {flag}")
+    assert flag == 0 and torch.isfinite(out).all() and err <= FWD_TOL and zerr <= 2.0 ** -13 * vmax + 1e-4
+
+
+@pytest.mark.parametrize("tau,causal", [(-0.5, True), (-2.0, False)])
+def test_negative_temperature_gradients(tau, causal):
+    """Both kernel families at a negative tau, forward and backward."""
+    from morphottention_amd import soft_morph_attention
+    B, N, H, m, dv = 1, 150, 2, 16, 64
+    x, params, dout = _inputs(B, N, H, m, dv, seed=1210)
+    ref_out, _, ref_grads = mo.soft_morph_ref_grads(x, *params, tau, H, m, scale=0.9, causal=causal, sgn=1, dout=dout,
+                                                    dtype=torch.float32)
+    for exact in (False, True):
+        leaves = [t.detach().clone().requires_grad_(True) for t in (x, *params)]
+        t = torch.tensor([tau], dtype=torch.float32, device="cuda", requires_grad=True)
+        out = soft_morph_attention(leaves[0], *leaves[1:], t, H, m, scale=0.9, causal=causal, exact=exact)
+        out.backward(dout)
+        err = ((out.float() - ref_out).abs() - _half_ulp(ref_out)).max().item()
+        rels = [((g.grad.float() - r.reshape(g.shape)).abs().max() / r.abs().max().clamp_min(1e-30)).item()
+                for g, r in zip((*leaves, t), ref_grads)]
+        _say(f"[soft] tau {tau} exact={exact}: beyond rounding {err:.2e} " +
+             " ".join(f"{n}={r:.2e}" for n, r in zip(NAMES, rels)))
+        assert err <= FWD_TOL and max(rels) <= GRAD_TOL
+
+
 def test_product_form_falls_back_for_small_tau():
     """tau = 0.02 spreads the exponents beyond the product form's range: the
     flag is raised and the element-wise kernels' result is returned as is."""
