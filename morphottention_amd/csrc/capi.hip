@@ -93,9 +93,10 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   // their values are stored as the zeros that the V^T layout wants there. (With
   // unpadded rows every value of a length that 8 does not divide was a 2-byte
   // store: proj_fwd at B64 N197 D768 H12 m64 142 us, padded 79 us with the same
-  // epilogue.) From 32 tokens on the padding is at most a quarter of the rows;
-  // shorter rows keep their own rows and the element stores.
-  d.NR = (int)(N >= 32 ? (N + 7) / 8 * 8 : N);
+  // epilogue; B2 N9 H8 m32 dv64 167 and 12.4, B1 N1 H1 m16 dv64 178 and 11.6.)
+  // A batch row's values take 3 NP D bytes of workspace, so TR stays far below
+  // 2^31 on any card.
+  d.NR = (int)((N + 7) / 8 * 8);
   d.TR = B * (int64_t)d.NR;
   d.D = (int)D;
   d.H = (int)H;
@@ -154,7 +155,7 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   if (NC % d.PBN == 0 && whole_heads(d.PBN)) {
     const int ntn = NC / d.PBN;
     // half-tile groups where both halves are whole 16-column blocks
-    const int half = d.NR % 8 == 0 && (d.HM / ntn) % 32 == 0 && (d.D / ntn) % 32 == 0 ? 2 : 1;
+    const int half = (d.HM / ntn) % 32 == 0 && (d.D / ntn) % 32 == 0 ? 2 : 1;
     d.PGW = d.PBN / half;
     d.PCPT = d.HM / ntn / half;
     d.PVPT = d.D / ntn / half;

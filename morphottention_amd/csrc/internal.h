@@ -16,8 +16,8 @@ struct Dims {
   int B, N, D, H, M, DV;  // batch, tokens, model dim, heads, cube_m, head_dim_v
   int NP;                 // N rounded up to a multiple of 64: row length of the V^T layout
   int64_t T;              // B * N tokens
-  int NR;                 // rows per batch row in the forward projection's row space: N, or N rounded up
-                          // to a multiple of 8 (make_dims)
+  int NR;                 // rows per batch row in the forward projection's row space: N rounded up to a
+                          // multiple of 8 (make_dims)
   int64_t TR;             // B * NR rows of that space
   int HM;                 // H * M projection columns
   int CW;                 // 2 * M + 8: code row width (hi/lo split codes + affine augmentation)

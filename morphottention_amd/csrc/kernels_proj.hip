@@ -168,7 +168,6 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
   const int nvw = min(G::WTN, NC - n0 - col0w);  // columns of this wave up to NC (the last tile of the natural order)
   static_assert(G::WN == 2, "half-tile groups are the two wave columns");
   const int lrow = lane >> 4, lcol = lane & 15;
-  const bool vec = d.NR % 8 == 0;
   // ---- values, straight from the accumulators: vt[bh][dd][n] = V_hi, and the
   // remainder V - V_hi as e4m3 in vlo's tile-major, key-permuted rows. A lane
   // holds 4 consecutive tokens of one column per 16-row block. Swapping 16-lane
@@ -176,7 +175,7 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
   // 16-byte piece of vt, 8 bytes of vlo); with four blocks, swapping 8-lane
   // halves between the two pairs then puts all 64 tokens of a column into one
   // store instruction (8 columns x 128 bytes of vt).
-  if (vec && ncode < BN) {
+  if (ncode < BN) {
     constexpr int NP2 = G::FI / 2;  // block pairs
     static_assert(NP2 == 1 || NP2 == 2, "wave rows of two or four blocks");
     const bool upper = NP2 == 2 && (lane & 8) != 0;
@@ -258,15 +257,12 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
       }
     }
   }
-  // columns that go through LDS: the codes, and the values of rows too short
-  // for whole groups of 8 tokens
-  const int nlds = vec ? ncode : min(BN, NC - n0);
-  if (nlds == 0) return;
+  if (ncode == 0) return;
 
   // ---- codes, through LDS: passes of 16 KB rows per wave row, 64 KB rows in
   // all (KB of the waves' 16-row blocks, as many as the main loop's LDS
   // holds), so that all the waves write and read in every pass.
-  const int SS = nlds + 4;  // row stride (floats): 16-byte rows, the accumulator stores on 64 distinct banks
+  const int SS = ncode + 4;  // row stride (floats): 16-byte rows, the accumulator stores on 64 distinct banks
   float* gtab = reinterpret_cast<float*>(smem);  // gate products G = gq gk of the code columns
   float* stage = gtab + BN;
   int lk = G::FI >= 4 ? 2 : G::FI >= 2 ? 1 : 0;  // log2 of the blocks per pass
@@ -280,10 +276,10 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
 #pragma unroll
     for (int i = 0; i < G::FI; ++i) {
       if (i >> lk != pass) continue;  // uniform
-      float* dst = stage + (64 * (i - (pass << lk)) + 16 * wm + 4 * lrow) * SS + (vec ? cw : col0w) + lcol;
+      float* dst = stage + (64 * (i - (pass << lk)) + 16 * wm + 4 * lrow) * SS + cw + lcol;
 #pragma unroll
       for (int j = 0; j < G::FJ; ++j)
-        if (16 * j < (vec ? ncw : nvw)) {  // uniform
+        if (16 * j < ncw) {  // uniform
 #pragma unroll
           for (int r = 0; r < 4; ++r) dst[r * SS + 16 * j] = acc[i][j][r];
         }
@@ -379,29 +375,6 @@ __global__ __launch_bounds__(kGemmThreads) void proj_fwd_kernel(const f16* __res
       *reinterpret_cast<f16x8*>(p.qa + bhn * CW + M) = f16x8{one, one, rh, rl, zero, zero, zero, zero};
       *reinterpret_cast<f16x8*>(p.ka + bhn * CW + M) = f16x8{bh_, bl_, one, one, zero, zero, zero, zero};
       p.tstat[bhn] = make_float4(bias, R, gap, t_ii);
-    }
-    if (!vec) {  // values one at a time
-      const int ntile = d.NP / 64;
-      for (int idx = tid; idx < (nlds - ncode) << lrows; idx += kGemmThreads) {
-        const int r = idx & ((1 << lrows) - 1), cc = ncode + (idx >> lrows);
-        const int t = m0 + G::WTM * ((r & 63) >> 4) + 16 * ((pass << lk) + (r >> 6)) + (r & 15);
-        if (t >= TR) continue;
-        const int b = t / d.NR, n = t - b * d.NR;  // NR == N here
-        const int vcol = d.PCPT > 0 ? tn * d.PVPT + cc - ncode : n0 + cc - d.HM, h = vcol / DV, dd = vcol % DV;
-        const int64_t bh = (int64_t)b * d.H + h;
-        const float x = stage[r * SS + cc];
-        const f16 vh = (f16)x;
-        f16* dst = p.vt + (bh * DV + dd) * d.NP + n;
-        uint8_t* low = p.vlo + ((bh * ntile + n / 64) * DV + dd) * 64;
-        dst[0] = vh;
-        const float vl[4] = {x - (float)vh, 0.f, 0.f, 0.f};
-        low[vlo_pos(n % 64)] = (uint8_t)vlo_pack4(vl);
-        if (n == d.N - 1)
-          for (int z = 1; n + z < d.NP; ++z) {
-            dst[z] = (f16)0.f;
-            low[vlo_pos((n + z) % 64)] = 0;
-          }
-      }
     }
   }
 }

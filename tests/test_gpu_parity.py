@@ -263,7 +263,7 @@ def test_projection_tile_128x160(B, N, D, H, causal):
 
 
 @pytest.mark.parametrize("B,N,H,m,dv", [
-    (3, 31, 2, 16, 64),      # short rows: unpadded, element stores
+    (3, 31, 2, 16, 64),      # padded to 32
     (3, 33, 2, 32, 64),      # padded to 40, 128-row tiles
     (5, 197, 3, 64, 64),     # padded to 200: batch rows change inside a tile
     (2, 71, 4, 16, 32),      # last group of one row of 8 with 7 live tokens
@@ -272,7 +272,12 @@ def test_projection_tile_128x160(B, N, D, H, causal):
     (52, 128, 5, 64, 64),    # heads must not straddle 160-column tiles
     (64, 199, 12, 64, 64),   # 128 x 256 tiles; backward GEMM tiles in 8 equal runs, cut inside a row panel
     (313, 128, 5, 64, 32),   # 128 x 256 tiles, natural column order, last column tile ragged
-], ids=["N31", "N33", "N197", "N71", "t320", "t256", "H5m64", "t128x256", "t128ragged"])
+    (2, 23, 4, 32, 32),      # short rows, each padded to 24: several batch rows in a group of 64
+    (9, 5, 5, 64, 64),       # padded to 8, one live group per batch row
+    (1024, 3, 32, 16, 64),   # 256 x 320 tiles of rows with 3 live tokens in 8
+    (2048, 2, 12, 64, 64),   # 128 x 256 tiles
+], ids=["N31", "N33", "N197", "N71", "t320", "t256", "H5m64", "t128x256", "t128ragged", "N23", "N5", "N3t320",
+        "N2t128x256"])
 def test_projection_rows_and_tiles(B, N, H, m, dv):
     """The projection's padded rows (N % 8 != 0), its tile shapes and column
     orders against the fp32 oracle."""
@@ -281,6 +286,35 @@ def test_projection_rows_and_tiles(B, N, H, m, dv):
     x, params, dout = make_inputs(B, N, D, H, m, seed=5100 + N)
     out, lse, grads = run_hip(x, params, H, m, m ** -0.5, False, dout)
     check(f"projection rows N={N} H={H} m={m}", out, lse, grads, *oracle(x, params, H, m, m ** -0.5, False, dout))
+
+
+@pytest.mark.parametrize("B,N,H,m,dv", [(1, 1, 1, 16, 64), (2, 9, 8, 32, 64), (64, 31, 4, 16, 128)])
+def test_short_ragged_rows_cost_no_more_than_whole_ones(B, N, H, m, dv):
+    """Rows of fewer than 32 tokens that 8 does not divide take the projection
+    about as long as the rows of the next multiple of 8, whose padded rows they
+    share (element stores had taken 3 to 14 times as long); 1.5 covers the
+    timing's noise."""
+    from morphottention_amd import capi
+
+    def proj_us(n):
+        x, params, _ = make_inputs(B, n, H * dv, H, m, seed=5200)
+        for _ in range(3):
+            torch.ops.morphottention.forward(x, *params, H, m, 1.0, False)
+        torch.cuda.synchronize()
+        capi.timing_only("proj_fwd")
+        capi.timing_enable(True)
+        capi.timing_read()
+        for _ in range(20):
+            torch.ops.morphottention.forward(x, *params, H, m, 1.0, False)
+        torch.cuda.synchronize()
+        t = sorted(ms for _, ms in capi.timing_read())
+        capi.timing_enable(False)
+        capi.timing_only(None)
+        return 1e3 * t[len(t) // 2]
+
+    ragged, whole = proj_us(N), proj_us((N + 7) // 8 * 8)
+    _say(f"[case] short rows B={B} N={N} H={H} m={m} dv={dv}: proj_fwd {ragged:.1f} us, whole groups {whole:.1f} us")
+    assert ragged <= 1.5 * whole
 
 
 @pytest.mark.parametrize("B,N,H,m,dv,causal", [
