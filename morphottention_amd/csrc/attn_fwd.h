@@ -24,9 +24,7 @@ __device__ __forceinline__ float sum8(const f16x8& v) {
 // 16 rows one b128 read phase touches land on distinct bank groups.
 __device__ __forceinline__ int vswz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// Launch shapes (SM), by how many workgroups the problem has (launch_attn_fwd_t).
-constexpr int kFwdRegular = 0, kFwdSmall = 1, kFwdSplit = 2;
-
+// SM: the launch shape (attn_fwd_shape)
 template <int M, int DV, int SM = kFwdRegular>
 struct FwdCfg {
   static constexpr int CW = 2 * M + 8;    // code row width
@@ -45,12 +43,11 @@ struct FwdCfg {
   // three per CU (LDS permitting), rather than one of eight waves; the waves
   // of a CU then wait at independent barriers (B1 N16384 H16 m32 causal:
   // forward -6 %; B16 N2048 H32 m64: -7 %).
-  static constexpr int QB2 = (M <= 32 && DV <= 64 && M * DV <= 1024) ? 2 : 1;
-  static constexpr bool HASSMALL = QB2 == 2 || (DV == 128 && M <= 32);  // else regular is small already
+  static constexpr int QB2 = fwd_two_blocks(M, DV) ? 2 : 1;
+  static constexpr bool HASSMALL = fwd_has_small(M, DV);
   static constexpr bool SMALL = SM != kFwdRegular && HASSMALL;
   static constexpr int QB = SMALL ? 1 : QB2;
   static constexpr bool W4 = QB2 == 1 && M >= 32 && DV <= 64;
-  static constexpr bool HASSPLIT = !(M == 64 && DV == 128);  // two groups' stages fit the LDS
   static constexpr int KS = SM == kFwdSplit ? 2 : 1;          // groups of WAVES waves
   static constexpr int WAVES = (SMALL || W4) ? 4 : 8 / QB;
   static constexpr int QW = 32 * QB * WAVES;  // 128 or 256 queries per workgroup
@@ -542,22 +539,14 @@ static hipError_t launch_attn_fwd_c(const Dims& d, const ProjBuffers& p, f16* ou
   return hipGetLastError();
 }
 
-// Launch shape. The split shape where the longest chain of tiles of one
-// workgroup is at least the mean work of a CU (few_long_chains): attn_fwd in us,
-// small or regular -> split, B1 H8 m16 dv64 N1024 15.9 -> 13.3, N2048 causal
-// 28.2 -> 22.7, B1 H16 N2048 31.3 -> 26.4, causal N3001 42.3 -> 33.6, N4096 59.6
-// -> 49.4; m64 B1 H8 N2048 causal 39.2 -> 32.8. Beyond: B8 H8 N1024 causal 18.9 ->
-// 20.6, unmasked B1 H16 N4096 90.1 -> 92.5. Small below two regular workgroups
-// per CU (m32 dv128, B1 H8 N2048 causal 54.4 -> 40.9; above that, at two per CU,
-// dv128 N4096 H16 135.6 -> 145.2).
 template <int M, int DV>
 static hipError_t launch_attn_fwd_t(const Dims& d, const ProjBuffers& p, f16* out, float* lse, hipStream_t s) {
-  using C = FwdCfg<M, DV>;
-  const int64_t bh = (int64_t)d.B * d.H;
-  if constexpr (C::HASSPLIT)
-    if (few_long_chains(d, 528)) return launch_attn_fwd_c<M, DV, kFwdSplit>(d, p, out, lse, s);
-  if constexpr (C::HASSMALL)
-    if ((d.N + C::QW - 1) / C::QW * bh < 2 * 256) return launch_attn_fwd_c<M, DV, kFwdSmall>(d, p, out, lse, s);
+  static_assert(FwdCfg<M, DV>::QW == 256 || !fwd_has_small(M, DV), "attn_fwd_shape counts regular workgroups of 256");
+  const int shape = attn_fwd_shape(d);
+  if constexpr (fwd_has_split(M, DV))
+    if (shape == kFwdSplit) return launch_attn_fwd_c<M, DV, kFwdSplit>(d, p, out, lse, s);
+  if constexpr (fwd_has_small(M, DV))
+    if (shape == kFwdSmall) return launch_attn_fwd_c<M, DV, kFwdSmall>(d, p, out, lse, s);
   return launch_attn_fwd_c<M, DV, kFwdRegular>(d, p, out, lse, s);
 }
 

@@ -84,27 +84,7 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   if ((causal & ~(15 | MORPHO_MODE_DETERMINISTIC)) != 0 || (causal & 12) == 12)
     return fail(MORPHO_ERR_INVALID_ARGUMENT,
                 "invalid mode bits 0x%x (causal | mask_diag | one projection | deterministic)", causal);
-  d.B = (int)B;
-  d.N = (int)N;
-  d.NP = (int)((N + 63) / 64 * 64);
-  // The projection's rows of one batch row are padded to whole groups of 8
-  // tokens, so that its epilogue writes V^T and the remainders of 8 tokens of
-  // one column at a time, whatever N is: the padding rows repeat a token and
-  // their values are stored as the zeros that the V^T layout wants there. (With
-  // unpadded rows every value of a length that 8 does not divide was a 2-byte
-  // store: proj_fwd at B64 N197 D768 H12 m64 142 us, padded 79 us with the same
-  // epilogue; B2 N9 H8 m32 dv64 167 and 12.4, B1 N1 H1 m16 dv64 178 and 11.6.)
-  // A batch row's values take 3 NP D bytes of workspace, so TR stays far below
-  // 2^31 on any card.
-  d.NR = (int)((N + 7) / 8 * 8);
-  d.TR = B * (int64_t)d.NR;
-  d.D = (int)D;
-  d.H = (int)H;
-  d.M = (int)M;
-  d.DV = (int)DV;
-  d.T = T;
-  d.HM = (int)(H * M);
-  d.CW = 2 * (int)M + 8;
+  fill_sizes(d, B, N, D, H, M);
   d.scale = scale;
   d.causal = causal & MORPHO_MODE_CAUSAL ? 1 : 0;
   d.mask_diag = causal & MORPHO_MODE_MASK_DIAG ? 1 : 0;
@@ -112,54 +92,7 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
            : causal & MORPHO_MODE_PROJ_IDENTITY ? kProjIdentity
                                                 : kProjSigmoid;
   d.det = causal & MORPHO_MODE_DETERMINISTIC ? 1 : 0;
-  // projection tiles: 256 x 320 when 320 divides H*M + D, else 256 x 256.
-  // When those would fill less than one round of the 256 CUs, 128-row tiles
-  // of 160 or 128 columns (whichever divides H*M + D and needs fewer rounds
-  // times tile area; 160 on a tie): e.g. H*M + D = 640, T = 8192 gives 256
-  // workgroups of 128 x 160 (one round) instead of 320 of 128 x 128. The
-  // interleaved column order needs whole heads and 16-column blocks per tile,
-  // and a tile whose width is no multiple of m (160 at m = 64) needs that order,
-  // or heads would straddle tiles.
-  const int NC = d.HM + d.D;
-  // tiles of bn columns (bn divides NC) can share the code and value columns
-  // evenly: whole heads and whole 16-column blocks each
-  auto whole_heads = [&](int bn) {
-    const int ntn = NC / bn;
-    return d.HM % ntn == 0 && d.D % ntn == 0 && (d.HM / ntn) % d.M == 0 && (d.D / ntn) % 16 == 0;
-  };
-  d.PBM = 256;
-  d.PBN = NC % 320 == 0 ? 320 : 256;
-  const int64_t rows = (d.TR + 127) / 128, big = (d.TR + 255) / 256 * ((NC + d.PBN - 1) / d.PBN);
-  if (big >= 256) {
-    // 128 x 256 tiles (one per CU, three stages) where their rounds, 0.58 of a
-    // 256 x 256 round each, are the shorter: a last round of few tiles costs
-    // half. proj_fwd in us, 256 -> 128 rows: B64 N197 D768 H12 m64 (300 tiles)
-    // 81 -> 69, B64 N256 78 -> 73, B1 N16384 D1024 H16 m32 92 -> 86, B4 N4096
-    // D1024 H8 m16 dv128 74 -> 68; the 320-wide tile has no such half.
-    const int64_t half = rows * ((NC + 255) / 256);
-    if (d.PBN == 256 && 100 * ((big + 255) / 256) > 58 * ((half + 255) / 256)) d.PBM = 128;
-  } else {
-    int64_t best = -1;
-    for (const int bn : {160, 128}) {
-      if (NC % bn || (bn % d.M && !whole_heads(bn))) continue;
-      const int64_t cost = (rows * (NC / bn) + 255) / 256 * bn;
-      if (best < 0 || cost < best) {
-        best = cost;
-        d.PBM = 128;
-        d.PBN = bn;
-      }
-    }
-  }
-  d.PGW = d.PBN;
-  d.PCPT = d.PVPT = 0;
-  if (NC % d.PBN == 0 && whole_heads(d.PBN)) {
-    const int ntn = NC / d.PBN;
-    // half-tile groups where both halves are whole 16-column blocks
-    const int half = (d.HM / ntn) % 32 == 0 && (d.D / ntn) % 32 == 0 ? 2 : 1;
-    d.PGW = d.PBN / half;
-    d.PCPT = d.HM / ntn / half;
-    d.PVPT = d.D / ntn / half;
-  }
+  choose_proj_tiles(d);
   return MORPHO_OK;
 }
 

@@ -6,43 +6,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "dispatch.h"
+
 namespace morpho {
-
-// Cube projections phi(z) (cube.cuh:9-17 of the reference): sigmoid (the
-// default), clamp((z + 1) / 2, 0, 1), and z itself.
-constexpr int kProjSigmoid = 0, kProjHardTanh01 = 1, kProjIdentity = 2;
-
-struct Dims {
-  int B, N, D, H, M, DV;  // batch, tokens, model dim, heads, cube_m, head_dim_v
-  int NP;                 // N rounded up to a multiple of 64: row length of the V^T layout
-  int64_t T;              // B * N tokens
-  int NR;                 // rows per batch row in the forward projection's row space: N rounded up to a
-                          // multiple of 8 (make_dims)
-  int64_t TR;             // B * NR rows of that space
-  int HM;                 // H * M projection columns
-  int CW;                 // 2 * M + 8: code row width (hi/lo split codes + affine augmentation)
-  float scale;
-  int causal;
-  int mask_diag;          // drop key j == query i
-  int proj;               // cube projection: kProjSigmoid, kProjHardTanh01 or kProjIdentity
-  int det;                // deterministic backward: dq and row sums from per-key-block partials
-  // Column order of the forward projection's B operand (wt rows): tiles of
-  // PBN columns in groups of PGW (whole or half tiles); when PCPT > 0 group g
-  // holds code columns [g PCPT, (g+1) PCPT) then value columns [g PVPT, (g+1)
-  // PVPT), so every tile (and, with half tiles, every wave) does the same
-  // epilogue work; PCPT == 0 keeps the natural order [W_phi | W_V].
-  int PBM, PBN, PGW, PCPT, PVPT;  // PBM: tile rows
-};
-
-// Whether the longest chain of 128-token blocks of one 128-token workgroup
-// (n128 of them) is at least the mean work of one of the 256 CUs: BH n128^2 / 256
-// blocks, or BH n128 (n128 + 1) / 512 under the causal mask (`causal_limit` for
-// BH (n128 + 1), about 512). The attention kernels then split each chain
-// between two groups of waves.
-inline bool few_long_chains(const Dims& d, int causal_limit) {
-  const int64_t bh = (int64_t)d.B * d.H, n128 = (d.N + 127) / 128;
-  return d.causal ? bh * (n128 + 1) <= causal_limit : bh * n128 <= 256;
-}
 
 // wt row (position in the projection's column order) of [W_phi | W_V] column c.
 __host__ __device__ inline int proj_row(const Dims& d, int c) {
@@ -126,24 +92,6 @@ hipError_t launch_bwd_gemm(const Dims& d, const ProjBuffers& p, const BwdBuffers
                            hipStream_t s);
 hipError_t launch_dw_reduce(const Dims& d, const BwdBuffers& g, const _Float16* gate_q, const _Float16* gate_k,
                             _Float16* dW_phi, _Float16* dW_V, _Float16* d_gate_q, _Float16* d_gate_k, hipStream_t s);
-// Work decomposition of the backward GEMM launch: one round of kGemmSlots
-// workgroups (the CUs of an MI355X; twice as many with 128 x 128 tiles, two
-// per CU). Workgroups [0, n_a), n_a / 8 per XCD (workgroup id % 8), compute g
-// whole dX tiles each; the next 8 ceil(tiles_w p / 8) each compute one piece
-// j < p of a dW tile t (the tile's kw token k-steps split into p near-equal
-// ranges; an XCD's workgroups take a contiguous run of the pieces in (j, t)
-// order, so they share token ranges). g and p are chosen so that both kinds take about the
-// same number of k-steps. Piece j stores an fp32 tile partial that dw_reduce
-// adds in piece order, so the result does not depend on timing.
-constexpr int kGemmSlots = 256;
-struct BwdGemmPlan {
-  int bt;                   // tile edge: 256, or 128 when that finishes sooner (few tiles)
-  int n_dx, ntn_x, kx;      // dX tiles, dX column tiles, k-steps per dX tile
-  int tiles_w, ntn_w, kw;   // dW tiles, dW column tiles, k-steps per dW tile (all tokens)
-  int g, n_a;               // dX tiles per type-A workgroup, type-A workgroups
-  int p;                    // pieces per dW tile (tiles_w p type-B workgroups and partials)
-};
-BwdGemmPlan bwd_gemm_plan(const Dims& d);
 // token k-step where piece j of a dW tile's kw k-steps starts (j = p: the end)
 __host__ __device__ inline int dw_piece_k0(int kw, int p, int j) { return (int)((int64_t)kw * j / p); }
 

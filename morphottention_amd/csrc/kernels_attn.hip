@@ -201,10 +201,8 @@ struct BwdCfg {
   static constexpr int MIN_WG = NW * NG == 4 ? 2 : 1;  // workgroups per CU (launch bound)
   static constexpr int OOFF = QT * QRB, AOFF = OOFF + QT * ORB;  // bytes
   static constexpr int STAGE = AOFF + 1024;
-  // LDS bytes: two stages and two dS^T tiles per group, the phi tile; whether
-  // the workgroup fits the CU (m = 64, dv = 128 split would spill 73 values)
-  static constexpr int STG = NG * 2 * STAGE, SDS = NG * 2 * KW * SRB, SPK = KW * PRB;
-  static constexpr bool FITS = STG + SDS + SPK <= 160 * 1024 && !(M == 64 && DV == 128);
+  // LDS bytes: two stages and two dS^T tiles per group, the phi tile
+  static constexpr int STG = NG * 2 * STAGE, SDS = NG * 2 * KW * SRB, SPK = KW * PRB, LDS = STG + SDS + SPK;
 };
 
 // Key-side (KV-outer) backward. A workgroup owns KW = 32 NW keys (32 per
@@ -872,17 +870,9 @@ static hipError_t launch_attn_bwd_h(const Dims& d, const ProjBuffers& p, const f
     if (!g.dqpart || !g.drpart) return hipErrorInvalidValue;
     return launch_attn_bwd_c<M, DV, HIOK, true, false>(d, p, grad_out, gate_q, gate_k, g, s);
   }
-  // The split shape where the longest chain of steps of one workgroup is at
-  // least the mean work of a CU (few_long_chains). attn_bwd in us, regular ->
-  // split: B1 H8 m32 dv64 N1024 43.7 -> 26.8, N2048 causal 81.3 -> 47.9, B1 H16
-  // causal N3001 m16 70.6 -> 52.3, m32 117 -> 87, B1 H16 N2048 m16 51.7 -> 41.9,
-  // m64 N2048 causal H8 116 -> 78, B2 H8 N1001 m32 dv128 54.8 -> 42.6. Beyond,
-  // the regular shape: unmasked B1 H16 N4096 m32 177 -> 217, causal B8 H8 N1024
-  // 55.3 -> 56.4 (dv 128); at m >= 32 it has eight waves on 256 keys and half
-  // the dq atomics (B1 H16 N4096 causal m64 225 -> 229, m32 157 -> 115), and
-  // two key blocks are too few steps (B8 H12 N197 m64 28.0 -> 30.4).
-  if constexpr (BwdCfg<M, DV, true>::FITS)
-    if (d.N > 256 && few_long_chains(d, M == 64 ? 420 : 528))
+  static_assert(BwdCfg<M, DV, true>::LDS <= 160 * 1024 || !bwd_has_split(M, DV), "the split shape must fit the LDS");
+  if constexpr (bwd_has_split(M, DV))
+    if (attn_bwd_split(d))
       return launch_attn_bwd_c<M, DV, HIOK, false, true>(d, p, grad_out, gate_q, gate_k, g, s);
   return launch_attn_bwd_c<M, DV, HIOK, false, false>(d, p, grad_out, gate_q, gate_k, g, s);
 }

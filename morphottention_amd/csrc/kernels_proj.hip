@@ -10,8 +10,6 @@
 //              reference drops, by symmetry),
 //             dX = [dZ | dV] [W_phi | W_V]^T,  [dW_phi | dW_V] = X^T [dZ | dV],
 //             gate gradients as deterministic fp32 column sums.
-#include <climits>
-
 #include "common.h"
 #include "gemm.h"
 #include "internal.h"
@@ -541,73 +539,6 @@ struct BwdTiles {
   static_assert(Dx::WN == Dw::WN && Dx::WTM == 64 && Dw::WTM == 64, "shared wave grid, 64-row wave tiles");
   static_assert(Dx::kBK == 64 && Dw::kBK == 64, "the plan counts k-steps of 64");
 };
-
-// Plan for tile edge bt and `slots` workgroups (the dW pieces take
-// 8 ceil(tiles_w p / 8) of them): for each g (dX tiles per type-A
-// workgroup), the most pieces p per dW tile that still fit the round,
-// scored by the longer of the two kinds: g kx against ceil(kw / p) k-steps
-// (plus one step of epilogue per dX tile or piece). When the dW tiles alone
-// fill the round, every workgroup takes one tile over several rounds. The dX
-// tiles, row panel by row panel, are dealt to the XCDs in 8 equal runs, so all
-// but the panels at a cut are read into one L2 (whole panels per XCD left
-// workgroups without a tile: 18 of 168 at B64 N197 D768 H12 m64, where the dW
-// pieces then took 50 k-steps instead of 40).
-static BwdGemmPlan plan_for(const Dims& d, int bt, int slots, int64_t& cost) {
-  BwdGemmPlan P;
-  const int NC = d.HM + d.D, T = (int)d.T;
-  P.bt = bt;
-  const int ntm_x = (T + bt - 1) / bt;
-  P.ntn_x = (d.D + bt - 1) / bt;
-  P.n_dx = ntm_x * P.ntn_x;
-  P.kx = (NC + 63) / 64;
-  P.ntn_w = (NC + bt - 1) / bt;
-  P.tiles_w = ((d.D + bt - 1) / bt) * P.ntn_w;
-  P.kw = (T + 63) / 64;
-  const int per_xcd = (P.n_dx + 7) / 8;  // dX tiles of one XCD
-  cost = INT64_MAX;
-  P.g = per_xcd;
-  P.n_a = 8;
-  P.p = 1;
-  for (int g = 1; g <= per_xcd; ++g) {
-    const int n_a = 8 * ((per_xcd + g - 1) / g);
-    int p = (slots - n_a) / P.tiles_w;
-    while (p > 0 && n_a + 8 * ((P.tiles_w * p + 7) / 8) > slots) --p;  // whole runs of 8
-    if (p < 1) continue;
-    p = p < P.kw ? p : P.kw;
-    const int64_t ca = (int64_t)g * (P.kx + 1), cb = (P.kw + p - 1) / p + 1;
-    const int64_t cst = ca > cb ? ca : cb;
-    if (cst < cost) {
-      cost = cst;
-      P.g = g;
-      P.n_a = n_a;
-      P.p = p;
-    }
-    if (ca > cost) break;  // g kx only grows from here
-  }
-  // no more pieces than the cost needs: each is a partial to write and add (B3
-  // N1500 D1024 H8 m32 dv128: 9 -> 4 pieces)
-  while (cost != INT64_MAX && P.p > 1 && (P.kw + P.p - 2) / (P.p - 1) + 1 <= cost) --P.p;
-  if (cost == INT64_MAX) {
-    // dW tiles alone fill the round: one dX tile or one whole dW tile per
-    // workgroup over several rounds (the dispatcher balances them)
-    P.g = 1;
-    P.n_a = 8 * per_xcd;
-    P.p = 1;
-    cost = ((int64_t)P.n_dx * (P.kx + 1) + (int64_t)P.tiles_w * (P.kw + 1) + slots - 1) / slots;
-  }
-  return P;
-}
-
-BwdGemmPlan bwd_gemm_plan(const Dims& d) {
-  int64_t c256, c128;
-  const BwdGemmPlan p256 = plan_for(d, 256, kGemmSlots, c256);
-  if (d.D % 128 != 0 || (d.HM + d.D) % 128 != 0) return p256;
-  // 128 x 128 tiles: two workgroups per CU (64 KiB of LDS each), so twice the
-  // slots; a k-step does a quarter of the work of a 256 x 256 one at about 2/3
-  // of its rate (more LDS and L2 traffic per MFMA), and shares its CU
-  const BwdGemmPlan p128 = plan_for(d, 128, 2 * kGemmSlots, c128);
-  return 3 * c128 < 4 * c256 ? p128 : p256;
-}
 
 struct BwdGemmArgs {
   const f16* X;

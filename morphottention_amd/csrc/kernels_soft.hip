@@ -359,11 +359,10 @@ __global__ __launch_bounds__(256) void soft_fvals_kernel(const f16* __restrict__
   }
 }
 
-// Four waves per column beyond one wave's first pass (512 keys).
 hipError_t launch_soft_fvals(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, const SoftState& st,
                              hipStream_t s) {
   const int ncol = d.B * d.H * d.DV;
-  if (d.NP > 512)
+  if (soft_fvals_waves(d) == 4)
     MORPHO_KLAUNCH(soft_fvals_kernel<4>, dim3((unsigned)ncol), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N, d.NP, d.DV,
                    ncol, (float)sgn);
   else
@@ -822,10 +821,7 @@ static hipError_t launch_soft_fwd_fast_t(const Dims& d, const ProjBuffers& p, co
 #define MORPHO_SOFT_TILE(MD_, SPLIT_)                                                                               \
   MORPHO_KLAUNCH((soft_fwd_tile_kernel<M, DV, MD_, SPLIT_>), grid, dim3(SPLIT_ ? 512 : 256), 0, s, p.qa, p.ka,      \
                  p.tstat, tau, st, out, zb, d.N, d.NP, d.H, d.D, d.B * d.H, d.causal, (float)sgn)
-    // the split shape as in the softmax forward. soft_fwd_fast in us, one group
-    // -> two: B2 N1001 H8 m32 29.0 -> 23.6, B1 N2048 H16 m16 50 -> 42, B1 H16
-    // causal N3000 m64 91 -> 71, N4096 m32 108 -> 91, B1 N300 H2 m16 11.3 -> 10.5
-    const bool split = few_long_chains(d, 528);
+    const bool split = soft_fwd_split(d);
     if (d.mask_diag && split)
       MORPHO_SOFT_TILE(true, true);
     else if (d.mask_diag)
@@ -1661,14 +1657,8 @@ static hipError_t launch_soft_bwd_fast_t(const Dims& d, const ProjBuffers& p, co
   MORPHO_KLAUNCH((soft_bwd_fast_kernel<M, DV, MD_, SPLIT_>), grid, dim3(SPLIT_ ? 512 : 256), 0, s, p.qa, p.ka, p.vt, \
                  p.vlo, p.tstat, tau, st, h, l, g.dq, g.dk, g.dcb, g.dzv, part, d.N, d.NP, d.H, d.D, d.HM,           \
                  d.B * d.H, d.causal, (float)sgn)
-  // as the softmax backward: the split shape where one workgroup's chain of
-  // steps is at least the mean work of a CU. soft_bwd_fast in us, regular ->
-  // split: B2 N1001 H8 m16 dv64 74 -> 55, m32 83 -> 60, m64 116 -> 77, B1 H16
-  // causal N3000 m16 170 -> 121, m64 272 -> 179, N4096 m32 274 -> 223; B1 N300 H2
-  // m16 32 -> 28. Two groups at dv = 128 would need more registers than two
-  // waves per SIMD have.
   if constexpr (DV <= 64) {
-    if (d.N > 256 && few_long_chains(d, 528)) {
+    if (soft_bwd_split(d)) {
       if (d.mask_diag)
         MORPHO_SOFT_BWD(true, true);
       else

@@ -1,0 +1,87 @@
+"""The launch rules of ``csrc/dispatch.h``, evaluated on the CPU.
+
+A small program prints, for one problem a line, what the rules choose:
+forward shape, the splits, the projection tiles and the backward GEMM plan.
+"""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+FIELDS = ("fwd", "bwd_split", "soft_fwd_split", "soft_bwd_split", "fvals_waves", "pbm", "pbn", "pgw", "pcpt", "pvpt",
+          "nr", "bt", "g", "n_a", "p", "tiles_w", "kw", "kx")
+PROGRAM = r'''
+#include <cstdio>
+#include "dispatch.h"
+using namespace morpho;
+int main() {
+  long long B, N, H, M, DV, causal, det;
+  while (scanf("%lld %lld %lld %lld %lld %lld %lld", &B, &N, &H, &M, &DV, &causal, &det) == 7) {
+    Dims d{};
+    d.causal = (int)causal;
+    d.det = (int)det;
+    fill_sizes(d, B, N, H * DV, H, M);
+    choose_proj_tiles(d);
+    const BwdGemmPlan P = bwd_gemm_plan(d);
+    printf("%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d\n", attn_fwd_shape(d), attn_bwd_split(d),
+           soft_fwd_split(d), soft_bwd_split(d), soft_fvals_waves(d), d.PBM, d.PBN, d.PGW, d.PCPT, d.PVPT, d.NR, P.bt,
+           P.g, P.n_a, P.p, P.tiles_w, P.kw, P.kx);
+  }
+}
+'''
+REGULAR, SMALL, SPLIT = 0, 1, 2
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """rules([(B, N, H, m, dv, causal), ...]) -> one dict of FIELDS per problem."""
+    d = tmp_path_factory.mktemp("dispatch")
+    (d / "rules.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{ROOT}/morphottention_amd/csrc",
+                    str(d / "rules.cpp"), "-o", str(d / "rules")], check=True)
+
+    def evaluate(problems):
+        text = "".join(" ".join(str(int(v)) for v in (*p, *([0] * (7 - len(p))))) + "\n" for p in problems)
+        out = subprocess.run([str(d / "rules")], input=text, capture_output=True, text=True, check=True).stdout
+        rows = [dict(zip(FIELDS, map(int, line.split()))) for line in out.splitlines()]
+        assert len(rows) == len(problems)
+        return rows
+
+    return evaluate
+
+
+def test_rules_at_measured_points(rules):
+    """The shapes at the configurations whose figures stand beside the rules."""
+    c2, c3, c4, c5, image = rules([(8, 1024, 8, 16, 64, False), (4, 4096, 16, 16, 64, True),
+                                   (1, 16384, 16, 32, 64, True), (16, 2048, 32, 64, 64, False),
+                                   (64, 197, 12, 64, 64, False)])
+    assert [r["fwd"] for r in (c2, c3, c4, c5, image)] == [SMALL, REGULAR, REGULAR, REGULAR, REGULAR]
+    assert not any(r[k] for r in (c2, c3, c4, c5, image) for k in ("bwd_split", "soft_fwd_split", "soft_bwd_split"))
+    assert [(r["pbm"], r["pbn"]) for r in (c2, c3, c4, c5, image)] == [
+        (128, 160), (256, 320), (128, 256), (256, 256), (128, 256)]
+    few, = rules([(1, 3001, 16, 16, 64, True)])
+    assert few["fwd"] == SPLIT and few["bwd_split"] and few["soft_fwd_split"] and few["soft_bwd_split"]
+    det, = rules([(1, 3001, 16, 16, 64, True, True)])
+    assert not det["bwd_split"]
+
+
+def test_projection_tiles_hold_whole_heads(rules):
+    """Every projection tile holds whole heads (a head's row sums are formed
+    within one tile), and rows are whole groups of 8 tokens."""
+    problems = [(B, N, H, m, dv, False) for B in (1, 9, 300) for N in (1, 5, 100, 197, 2048)
+                for H in (1, 2, 3, 5, 6, 7, 8, 12, 16, 20, 24, 32) for m in (16, 32, 64) for dv in (32, 64, 128)]
+    for (B, N, H, m, dv, _), r in zip(problems, rules(problems)):
+        assert r["nr"] == (N + 7) // 8 * 8
+        if r["pcpt"]:
+            groups = r["pbn"] // r["pgw"]
+            assert r["pcpt"] * groups % m == 0 and r["pcpt"] % 16 == 0 and r["pvpt"] % 16 == 0
+            assert (r["pcpt"] + r["pvpt"]) == r["pgw"]
+        else:
+            assert r["pbn"] % m == 0
