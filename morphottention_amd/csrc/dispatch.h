@@ -169,8 +169,26 @@ inline bool soft_fwd_split(const Dims& d) { return d.DV <= 64 && few_long_chains
 // waves per SIMD have.
 inline bool soft_bwd_split(const Dims& d) { return d.DV <= 64 && d.N > 256 && few_long_chains(d, 528); }
 
-// Waves per value column of soft_fvals: four beyond one wave's first pass (512 keys).
-inline int soft_fvals_waves(const Dims& d) { return d.NP > 512 ? 4 : 1; }
+// Lanes per value column of soft_fvals, 8 keys each: as many as the column has
+// groups of 8, up to a wave; a workgroup of four waves for few long columns,
+// which would leave most of the chip idle. soft_fvals in us, one wave -> four:
+// 64 columns N4096 8.4 -> 4.2, 1024 columns N2048 6.0 -> 5.2, N4096 9.8 -> 7.8;
+// 2048 columns N2048 7.5 -> 7.5, N4096 13.9 -> 14.3; 8192 columns N4096 53 -> 61,
+// N513 10.2 -> 13.9; 32768 columns N513 31 -> 45. Short columns, one wave -> 8
+// lanes: 131072 columns N16 69 -> 11.4.
+inline int soft_fvals_lanes(const Dims& d) {
+  if (d.NP <= 64) return 8;
+  if (d.NP <= 128) return 16;
+  if (d.NP <= 256) return 32;
+  return d.NP > 1024 && (int64_t)d.B * d.D < 2048 ? 256 : 64;
+}
+// Its workgroups of 256 lanes, which take further columns in turn beyond 2^20:
+// one lane group for every column would pass 2^32 work-items within the
+// accepted sizes (B D = 2^24 columns of 256 lanes).
+inline unsigned soft_fvals_grid(const Dims& d) {
+  const int64_t per = 256 / soft_fvals_lanes(d), wgs = ((int64_t)d.B * d.D + per - 1) / per;
+  return (unsigned)(wgs < (1 << 20) ? wgs : 1 << 20);
+}
 
 // Work decomposition of the backward GEMM launch: one round of kGemmSlots
 // workgroups (the CUs of an MI355X; twice as many with 128 x 128 tiles, two

@@ -294,80 +294,88 @@ constexpr float kProductFloor = 0x1p-80f;
 // (the column reference B_c is kw max V for kw > 0, kw min V for kw < 0), then
 // F^T = 2^(w - B_c) of its keys as bf16 hi / lo pairs, [B*H, DV, NP] with keys
 // contiguous: the tiles every query block of the product-form forward reads.
-// WPC waves per column, 8 keys per lane and pass; the second pass over V reads
-// lines that the first just brought in. Bound by HBM (3 bytes read and 4
-// written per value). As two launches: 9.0 + 20.6 us at B4 N4096 H16 dv64, 4.0 +
-// 4.4 at B2 N1001 H8 dv64; now 28.4 and 4.4. Block 0 also clears the fallback
-// flag of this call.
-template <int WPC>
+// LPC lanes per column (soft_fvals_lanes), 8 keys per lane and pass; the second
+// pass over V reads lines that the first just brought in. Bound by HBM (3 bytes
+// read and 4 written per value). As two launches: 9.0 + 20.6 us at B4 N4096 H16
+// dv64, 4.0 + 4.4 at B2 N1001 H8 dv64; now 26.3 and 4.5. Block 0 also clears
+// the fallback flag of this call.
+template <int LPC>
 __global__ __launch_bounds__(256) void soft_fvals_kernel(const f16* __restrict__ vt, const uint8_t* __restrict__ vlo,
                                                          const float* __restrict__ tau_p, SoftState st, int N, int NP,
                                                          int DV, int ncol, float sgn) {
   __shared__ float ext[2][4];
   if (blockIdx.x == 0 && threadIdx.x == 0) *st.flag = 0;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int col = WPC == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
-  const int first = 8 * (WPC == 1 ? lane : (int)threadIdx.x), step = 512 * WPC;
-  if (col >= ncol) return;  // uniform over the column's waves
-  const int bh = col / DV, c = col - bh * DV;
-  float hi = kNegInf, lo = -kNegInf;
-  for (int k0 = first; k0 < N; k0 += step) {
-    float v[8];
-    load_values8(vt, vlo, bh, DV, NP, c, k0, v);
+  constexpr int kCols = 256 / LPC, step = 8 * LPC;  // columns of a workgroup, keys of a pass
+  const int first = 8 * ((int)threadIdx.x % LPC);
+  // uniform over a column's lanes; at LPC = 256 there is a workgroup for every column
+  for (int col = (int)blockIdx.x * kCols + (int)threadIdx.x / LPC; col < ncol; col += (int)gridDim.x * kCols) {
+    const int bh = col / DV, c = col - bh * DV;
+    float hi = kNegInf, lo = -kNegInf;
+    for (int k0 = first; k0 < N; k0 += step) {
+      float v[8];
+      load_values8(vt, vlo, bh, DV, NP, c, k0, v);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (k0 + j < N) {
-        hi = fmaxf(hi, v[j]);
-        lo = fminf(lo, v[j]);
+      for (int j = 0; j < 8; ++j) {
+        const bool in = k0 + j < N;
+        hi = in ? fmaxf(hi, v[j]) : hi;
+        lo = in ? fminf(lo, v[j]) : lo;
       }
-  }
-#pragma unroll
-  for (int sh = 32; sh >= 1; sh >>= 1) {
-    hi = fmaxf(hi, __shfl_xor(hi, sh));
-    lo = fminf(lo, __shfl_xor(lo, sh));
-  }
-  if constexpr (WPC == 4) {
-    if (lane == 0) {
-      ext[0][wv] = hi;
-      ext[1][wv] = lo;
     }
-    __syncthreads();
-    hi = fmaxf(fmaxf(ext[0][0], ext[0][1]), fmaxf(ext[0][2], ext[0][3]));
-    lo = fminf(fminf(ext[1][0], ext[1][1]), fminf(ext[1][2], ext[1][3]));
-  }
-  if (first == 0) {
-    st.vmax[col] = hi;
-    st.vmin[col] = lo;
-  }
-  const float kw = sgn * kLog2e / *tau_p;
-  const float bc = kw * (kw > 0.f ? hi : lo);
-  for (int k0 = first; k0 < NP; k0 += step) {
-    bf16x8 fh, fl;
-    float v[8];
-    load_values8(vt, vlo, bh, DV, NP, c, k0, v);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float ev = fast_exp2(kw * v[j] - bc);
-      const float f = k0 + j < N ? ev : 0.f;
-      bf16 h, l;
-      split_bf16(f, h, l);
-      fh[j] = h;
-      fl[j] = l;
+    for (int sh = 1; sh < (LPC < 64 ? LPC : 64); sh *= 2) {
+      hi = fmaxf(hi, __shfl_xor(hi, sh));
+      lo = fminf(lo, __shfl_xor(lo, sh));
     }
-    *reinterpret_cast<bf16x8*>(st.fth + (int64_t)col * NP + k0) = fh;
-    *reinterpret_cast<bf16x8*>(st.ftl + (int64_t)col * NP + k0) = fl;
+    if constexpr (LPC == 256) {
+      if (lane == 0) {
+        ext[0][wv] = hi;
+        ext[1][wv] = lo;
+      }
+      __syncthreads();
+      hi = fmaxf(fmaxf(ext[0][0], ext[0][1]), fmaxf(ext[0][2], ext[0][3]));
+      lo = fminf(fminf(ext[1][0], ext[1][1]), fminf(ext[1][2], ext[1][3]));
+    }
+    if (first == 0) {
+      st.vmax[col] = hi;
+      st.vmin[col] = lo;
+    }
+    const float kw = sgn * kLog2e / *tau_p;
+    const float bc = kw * (kw > 0.f ? hi : lo);
+    for (int k0 = first; k0 < NP; k0 += step) {
+      bf16x8 fh, fl;
+      float v[8];
+      load_values8(vt, vlo, bh, DV, NP, c, k0, v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float ev = fast_exp2(kw * v[j] - bc);
+        const float f = k0 + j < N ? ev : 0.f;
+        bf16 h, l;
+        split_bf16(f, h, l);
+        fh[j] = h;
+        fl[j] = l;
+      }
+      *reinterpret_cast<bf16x8*>(st.fth + (int64_t)col * NP + k0) = fh;
+      *reinterpret_cast<bf16x8*>(st.ftl + (int64_t)col * NP + k0) = fl;
+    }
+    if constexpr (LPC == 256) return;  // no second column: ext is in use
   }
 }
 
 hipError_t launch_soft_fvals(const Dims& d, const ProjBuffers& p, const float* tau, int sgn, const SoftState& st,
                              hipStream_t s) {
-  const int ncol = d.B * d.H * d.DV;
-  if (soft_fvals_waves(d) == 4)
-    MORPHO_KLAUNCH(soft_fvals_kernel<4>, dim3((unsigned)ncol), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N, d.NP, d.DV,
-                   ncol, (float)sgn);
-  else
-    MORPHO_KLAUNCH(soft_fvals_kernel<1>, dim3((unsigned)((ncol + 3) / 4)), dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N,
-                   d.NP, d.DV, ncol, (float)sgn);
+  const int ncol = d.B * d.D;  // below 2^31: a column has 7 NP bytes of workspace
+  const dim3 grid(soft_fvals_grid(d));
+#define MORPHO_FVALS(LPC_)                                                                                           \
+  MORPHO_KLAUNCH(soft_fvals_kernel<LPC_>, grid, dim3(256), 0, s, p.vt, p.vlo, tau, st, d.N, d.NP, d.DV, ncol, (float)sgn)
+  switch (soft_fvals_lanes(d)) {
+    case 8: MORPHO_FVALS(8); break;
+    case 16: MORPHO_FVALS(16); break;
+    case 32: MORPHO_FVALS(32); break;
+    case 64: MORPHO_FVALS(64); break;
+    default: MORPHO_FVALS(256);
+  }
+#undef MORPHO_FVALS
   return hipGetLastError();
 }
 

@@ -13,7 +13,7 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-FIELDS = ("fwd", "bwd_split", "soft_fwd_split", "soft_bwd_split", "fvals_waves", "pbm", "pbn", "pgw", "pcpt", "pvpt",
+FIELDS = ("fwd", "bwd_split", "soft_fwd_split", "soft_bwd_split", "fvals_lanes", "fvals_grid", "pbm", "pbn", "pgw", "pcpt", "pvpt",
           "nr", "bt", "g", "n_a", "p", "tiles_w", "kw", "kx")
 PROGRAM = r'''
 #include <cstdio>
@@ -28,8 +28,8 @@ int main() {
     fill_sizes(d, B, N, H * DV, H, M);
     choose_proj_tiles(d);
     const BwdGemmPlan P = bwd_gemm_plan(d);
-    printf("%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d\n", attn_fwd_shape(d), attn_bwd_split(d),
-           soft_fwd_split(d), soft_bwd_split(d), soft_fvals_waves(d), d.PBM, d.PBN, d.PGW, d.PCPT, d.PVPT, d.NR, P.bt,
+    printf("%d %d %d %d %d %u %d %d %d %d %d %d %d %d %d %d %d %d %d\n", attn_fwd_shape(d), attn_bwd_split(d),
+           soft_fwd_split(d), soft_bwd_split(d), soft_fvals_lanes(d), soft_fvals_grid(d), d.PBM, d.PBN, d.PGW, d.PCPT, d.PVPT, d.NR, P.bt,
            P.g, P.n_a, P.p, P.tiles_w, P.kw, P.kx);
   }
 }
@@ -85,3 +85,17 @@ def test_projection_tiles_hold_whole_heads(rules):
             assert (r["pcpt"] + r["pvpt"]) == r["pgw"]
         else:
             assert r["pbn"] % m == 0
+
+
+def test_soft_fvals_grid_at_the_limits(rules):
+    """The launch covers every column and stays below 2^31 work-items at every
+    accepted size (one 256-lane workgroup per column had passed 2^32 from B D =
+    2^24 on; B8192 N513 D2048 fits an MI355X)."""
+    problems = [(8192, 513, 32, 16, 64, False), (1 << 25, 1, 1, 16, 32, False), (1 << 17, 600, 2, 16, 64, True),
+                (1 << 20, 64, 16, 16, 64, False), (4, 4096, 16, 16, 64, True), (2, 1001, 8, 32, 64, False),
+                (1, 1, 1, 16, 32, False), (3, 65, 5, 64, 128, True), (7, 200, 3, 16, 32, False)]
+    for (B, N, H, m, dv, _), r in zip(problems, rules(problems)):
+        cols = 256 // r["fvals_lanes"]
+        assert 0 < r["fvals_grid"] * 256 < 2 ** 31
+        assert r["fvals_grid"] * cols >= B * H * dv or r["fvals_grid"] == 1 << 20
+        assert r["fvals_grid"] * cols - cols < B * H * dv

@@ -136,7 +136,8 @@ def test_soft_ragged_lengths(N):
     (63, 16, 32, False, 1), (64, 16, 64, True, -1), (65, 32, 64, False, -1),   # one tile, and one key of a second
     (128, 64, 64, True, 1), (129, 64, 32, True, -1), (193, 32, 32, True, 1),   # both stage counts, masked tails
     (400, 64, 64, False, -1), (333, 16, 32, False, 1),       # with the split backward: odd numbers of steps
-    (290, 64, 32, True, 1), (385, 16, 64, True, -1), (257, 32, 64, False, 1)])
+    (290, 64, 32, True, 1), (385, 16, 64, True, -1), (257, 32, 64, False, 1),
+    (1030, 16, 32, True, 1)])                                # four waves per value column
 def test_soft_forward_tiles(N, m, dv, causal, sgn):
     """The 64-key tiles of the product-form forward (dv <= 64) at their edges,
     and from 257 tokens on the split shape of its backward."""
@@ -145,6 +146,16 @@ def test_soft_forward_tiles(N, m, dv, causal, sgn):
     x, params, dout = _inputs(B, N, H, m, dv, seed=7000 + N)
     out, zb, grads = _run(x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
     _check(f"soft tiles N={N}", out, zb, grads, x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
+
+
+def test_soft_values_of_many_long_columns():
+    """From 2048 value columns on, columns of more than 512 keys keep one wave
+    of several passes."""
+    B, N, H, m, dv = 8, 577, 8, 16, 32
+    _say(f"[case] soft many columns B={B} N={N} H={H} m={m} dv={dv}")
+    x, params, dout = _inputs(B, N, H, m, dv, seed=7100)
+    out, zb, grads = _run(x, params, 0.6, H, m, 0.25, True, -1, dout)
+    _check("soft many columns", out, zb, grads, x, params, 0.6, H, m, 0.25, True, -1, dout)
 
 
 def test_soft_variants_masked_diagonal_and_projection():
