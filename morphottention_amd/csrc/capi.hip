@@ -73,10 +73,10 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   // token, the deterministic dq reduction one per 4 (token, head, code)
   // values; the bounds below keep each under 2^31. They sit near what fits in
   // memory anyway (T D = 2^34 is a 32 GiB fp16 input).
-  if (B > ((int64_t)1 << 28) || N > ((int64_t)1 << 28))
+  if (B > kMaxTokens || N > kMaxTokens)
     return fail(MORPHO_ERR_INVALID_ARGUMENT, "problem too large: B * N must be at most 2^28 tokens");
   const int64_t T = B * N;
-  if (T > ((int64_t)1 << 28) || D > 65536 || H * M > 65536 || T * D > ((int64_t)1 << 34) ||
+  if (T > kMaxTokens || D > 65536 || H * M > 65536 || T * D > ((int64_t)1 << 34) ||
       T * H * M > ((int64_t)1 << 33))
     return fail(MORPHO_ERR_INVALID_ARGUMENT,
                 "problem too large: needs B*N <= 2^28, B*N*D <= 2^34, B*N*H*cube_m <= 2^33, D and H*cube_m <= 65536");

@@ -12,6 +12,9 @@ namespace morpho {
 // default), clamp((z + 1) / 2, 0, 1), and z itself.
 constexpr int kProjSigmoid = 0, kProjHardTanh01 = 1, kProjIdentity = 2;
 
+// Most tokens B N of a call (make_dims refuses more).
+constexpr int64_t kMaxTokens = (int64_t)1 << 28;
+
 struct Dims {
   int B, N, D, H, M, DV;  // batch, tokens, model dim, heads, cube_m, head_dim_v
   int NP;                 // N rounded up to a multiple of 64: row length of the V^T layout

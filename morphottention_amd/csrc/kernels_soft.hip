@@ -614,7 +614,9 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
   const float ks = 1.f / fabsf(tau), kw = sgn * kLog2e / tau;
   for (int c = tid; c < DV; c += 256) sbc[c] = kw * (kw > 0.f ? st.vmax[bh * DV + c] : st.vmin[bh * DV + c]);
 
-  // ---- DMA: per-lane byte offsets of this wave's chunks, computed once
+  // ---- DMA: per-lane byte offsets of this wave's chunks, computed once (an F^T
+  // chunk's from its own first row: 7 rows on, they fit 32 bits at every length)
+  static_assert((7 * kMaxTokens + C::KT) * 2 < (int64_t)1 << 32, "F^T lane offsets must fit 32 bits");
   const f16* const fth = reinterpret_cast<const f16*>(st.fth) + fbase;
   const f16* const ftl = reinterpret_cast<const f16*>(st.ftl) + fbase;
   const unsigned sbase = (unsigned)(uintptr_t)(__attribute__((address_space(3))) f16*)smem;
@@ -628,7 +630,7 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
 #pragma unroll
   for (int j = 0; j < C::NFW; ++j) {
     const int v = (w + C::WAVES * j) % C::FCH, r = 8 * v + (lane >> 3);
-    foff[j] = (unsigned)(((int64_t)r * NP + 8 * ((lane & 7) ^ fswz(r))) * 2);
+    foff[j] = (unsigned)(((int64_t)(lane >> 3) * NP + 8 * ((lane & 7) ^ fswz(r))) * 2);
   }
   auto issue = [&](int t) {
     const unsigned dst = sbase + 2u * (unsigned)((t % C::NSTAGE) * C::STAGE);
@@ -649,7 +651,8 @@ soft_fwd_tile_kernel(const f16* __restrict__ qa, const f16* __restrict__ ka, con
 #pragma unroll
     for (int j = 0; j < C::NFW; ++j) {  // zero from N to NP >= k0 + KT
       const int v = w + C::WAVES * j;
-      lds_dma16_so((v < C::FCH ? fth : ftl) + k0, foff[j], dst + 2u * C::FOFF + 1024u * (unsigned)v);
+      lds_dma16_so((v < C::FCH ? fth : ftl) + (int64_t)(8 * (v % C::FCH)) * NP + k0, foff[j],
+                   dst + 2u * C::FOFF + 1024u * (unsigned)v);
     }
   };
 
