@@ -116,10 +116,17 @@ inline void choose_proj_tiles(Dims& d) {
 // (n128 of them) is at least the mean work of one of the 256 CUs: BH n128^2 / 256
 // blocks, or BH n128 (n128 + 1) / 512 under the causal mask (`causal_limit` for
 // BH (n128 + 1), about 512). The attention kernels then split each chain
-// between two groups of waves.
-inline bool few_long_chains(const Dims& d, int causal_limit) {
+// between two groups of waves, one workgroup per CU. Under the causal mask
+// there can be more than 256 workgroups; without the long chains that the
+// second round's short ones fill up behind, that second round costs more than
+// the split gains: attn_fwd in us, not split -> split, causal, 352 workgroups of
+// N256 m32 dv64 9.8 -> 15.5, 384 of N512 13.7 -> 16.7, of N640 15.8 -> 18.6, of N768
+// 17.4 -> 18.4 (up to 256 workgroups N512 0.92 to 0.97 of the time, beyond N1000
+// 0.90 with either).
+inline bool few_long_chains(const Dims& d, int causal_limit, bool two_short_rounds = false) {
   const int64_t bh = (int64_t)d.B * d.H, n128 = (d.N + 127) / 128;
-  return d.causal ? bh * (n128 + 1) <= causal_limit : bh * n128 <= 256;
+  if (!d.causal) return bh * n128 <= 256;
+  return bh * (n128 + 1) <= causal_limit && (bh * n128 <= 256 || n128 > 6 || two_short_rounds);
 }
 
 // Launch shapes of the attention forward.
@@ -135,11 +142,14 @@ constexpr bool fwd_has_split(int M, int DV) { return !(M == 64 && DV == 128); } 
 // small or regular -> split, B1 H8 m16 dv64 N1024 15.9 -> 13.3, N2048 causal
 // 28.2 -> 22.7, B1 H16 N2048 31.3 -> 26.4, causal N3001 42.3 -> 33.6, N4096 59.6
 // -> 49.4; m64 B1 H8 N2048 causal 39.2 -> 32.8. Beyond: B8 H8 N1024 causal 18.9 ->
-// 20.6, unmasked B1 H16 N4096 90.1 -> 92.5. Small below two regular workgroups
-// per CU (m32 dv128, B1 H8 N2048 causal 54.4 -> 40.9; above that, at two per CU,
-// dv128 N4096 H16 135.6 -> 145.2).
+// 20.6, unmasked B1 H16 N4096 90.1 -> 92.5. From four key tiles on, six where the
+// other shape has 128 queries per workgroup anyway (mean time against not
+// split, at N64 1.04 and 1.11, N128 1.03 and 1.10, N256 0.99 and 1.04, N385 0.95 and
+// 0.99). Small below two regular workgroups per CU (m32 dv128, B1 H8 N2048 causal
+// 54.4 -> 40.9; above that, at two per CU, dv128 N4096 H16 135.6 -> 145.2).
 inline int attn_fwd_shape(const Dims& d) {
-  if (fwd_has_split(d.M, d.DV) && few_long_chains(d, 528)) return kFwdSplit;
+  const int most_unsplit = fwd_has_small(d.M, d.DV) ? 192 : 320;
+  if (fwd_has_split(d.M, d.DV) && d.N > most_unsplit && few_long_chains(d, 528)) return kFwdSplit;
   if (fwd_has_small(d.M, d.DV) && (int64_t)((d.N + 255) / 256) * d.B * d.H < 2 * 256) return kFwdSmall;
   return kFwdRegular;
 }
@@ -155,15 +165,19 @@ constexpr bool bwd_has_split(int M, int DV) { return DV <= 64 || M == 32; }
 // the regular shape: unmasked B1 H16 N4096 m32 177 -> 217, causal B8 H8 N1024
 // 55.3 -> 56.4 (dv 128); at m >= 32 it has eight waves on 256 keys and half
 // the dq atomics (B1 H16 N4096 causal m64 225 -> 229, m32 157 -> 115), and
-// two key blocks are too few steps (B8 H12 N197 m64 28.0 -> 30.4).
+// two key blocks are too few steps (B8 H12 N197 m64 28.0 -> 30.4). Two short
+// rounds still gain where the regular shape has eight waves (384 workgroups of
+// causal N384: m32 dv64 -10 % or more, m16 dv64 +13 %, m32 dv128 +15 %).
 inline bool attn_bwd_split(const Dims& d) {
-  return bwd_has_split(d.M, d.DV) && !d.det && d.N > 256 && few_long_chains(d, d.M == 64 ? 420 : 528);
+  return bwd_has_split(d.M, d.DV) && !d.det && d.N > 256 &&
+         few_long_chains(d, d.M == 64 ? 420 : 528, d.M >= 32 && d.DV <= 64);
 }
 
 // The split shape as in the softmax forward. soft_fwd_fast in us, one group
 // -> two: B2 N1001 H8 m32 29.0 -> 23.6, B1 N2048 H16 m16 50 -> 42, B1 H16
-// causal N3000 m64 91 -> 71, N4096 m32 108 -> 91, B1 N300 H2 m16 11.3 -> 10.5
-inline bool soft_fwd_split(const Dims& d) { return d.DV <= 64 && few_long_chains(d, 528); }
+// causal N3000 m64 91 -> 71, N4096 m32 108 -> 91, B1 N300 H2 m16 11.3 -> 10.5;
+// with one key tile +5 %, with two 0 to -10 %.
+inline bool soft_fwd_split(const Dims& d) { return d.DV <= 64 && d.N > 64 && few_long_chains(d, 528); }
 // As the softmax backward: the split shape where one workgroup's chain of
 // steps is at least the mean work of a CU. soft_bwd_fast in us, regular ->
 // split: B2 N1001 H8 m16 dv64 74 -> 55, m32 83 -> 60, m64 116 -> 77, B1 H16

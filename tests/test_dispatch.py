@@ -99,3 +99,33 @@ def test_soft_fvals_grid_at_the_limits(rules):
         assert 0 < r["fvals_grid"] * 256 < 2 ** 31
         assert r["fvals_grid"] * cols >= B * H * dv or r["fvals_grid"] == 1 << 20
         assert r["fvals_grid"] * cols - cols < B * H * dv
+
+
+def test_gpu_parity_cases_run_the_shapes_they_name(rules):
+    from test_gpu_parity import LAUNCH_SHAPES
+    for case, r in zip(LAUNCH_SHAPES, rules([c[:6] for c in LAUNCH_SHAPES])):
+        assert (("regular", "small", "split")[r["fwd"]], "split" if r["bwd_split"] else "regular") == case[6:], case
+
+
+def test_split_shapes_stay_where_they_gain(rules):
+    """No split forward for the few key tiles where one group is as fast, and no
+    second round of one-per-CU workgroups for short causal chains (measured up
+    to 1.2 and 1.6 times the time without)."""
+    def workgroups(case):
+        return case[0] * case[2] * ((case[1] + 127) // 128)
+
+    short = [(1, N, H, m, dv, c) for N in (1, 33, 64, 100, 128, 192) for H in (1, 8) for m in (16, 32, 64)
+             for dv in (32, 64, 128) for c in (False, True)]
+    for case, r in zip(short, rules(short)):
+        assert r["fwd"] != SPLIT and not r["bwd_split"] and not r["soft_bwd_split"], case
+        assert r["soft_fwd_split"] == (case[1] > 64 and case[4] <= 64), case
+    rounds = [(B, N, 8, m, dv, True) for N in (193, 256, 300, 384, 512, 640, 768) for B in range(5, 23)
+              for m in (16, 32, 64) for dv in (32, 64, 128)]
+    for case, r in zip(rounds, rules(rounds)):
+        if workgroups(case) > 256:
+            assert r["fwd"] != SPLIT and not r["soft_fwd_split"] and not r["soft_bwd_split"], case
+            assert not r["bwd_split"] or (case[3] >= 32 and case[4] <= 64), case
+    long = [(1, N, H, m, dv, c) for N in (1000, 3000) for H in (8, 10) for m in (16, 32, 64) for dv in (32, 64)
+            for c in (False, True)]
+    assert all(r["fwd"] == SPLIT and r["bwd_split"] and r["soft_fwd_split"] and r["soft_bwd_split"]
+               for r in rules(long))

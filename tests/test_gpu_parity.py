@@ -317,28 +317,42 @@ def test_short_ragged_rows_cost_no_more_than_whole_ones(B, N, H, m, dv):
     assert ragged <= 1.5 * whole
 
 
-@pytest.mark.parametrize("B,N,H,m,dv,causal", [
-    (1, 40, 1, 16, 64, False),     # split, one tile: the second group has none
-    (1, 65, 2, 32, 32, True),      # split, a second tile of one key
-    (1, 1000, 3, 16, 32, True),    # split, odd number of tiles
-    (2, 900, 2, 64, 64, False),    # split, ragged
-    (1, 700, 2, 32, 128, True),    # split, wide heads
-    (1, 2500, 20, 16, 64, True),   # split up to two workgroups per CU
-    (5, 900, 8, 16, 128, False),   # small shape of wide heads
-    (9, 300, 16, 32, 128, True),   # small, waves past the last query
-    (2, 257, 2, 16, 64, True),     # split backward: three key blocks, one key in the last
-    (1, 288, 3, 64, 32, False),    # split backward, nine steps: one more for the first group
-    (1, 1100, 2, 64, 64, True),    # split backward, two dq tiles per wave
-    (44, 300, 2, 32, 64, True),    # regular backward, eight waves on 256 keys
-    (44, 300, 2, 64, 32, True),
-    (44, 300, 2, 64, 64, False),
-], ids=lambda v: str(v))
-def test_launch_shapes(B, N, H, m, dv, causal):
-    """The split and small launch shapes of the forward and the split shape of
-    the backward against the oracle, on the reference path (default gates) and the exact-maximum path (signed
-    gates; 2 sigma keeps the scores of m = 64 in the fp32 oracle's range)."""
+# (B, N, H, m, dv, causal, forward shape, backward shape); tests/test_dispatch.py
+# checks that the launch rules give these shapes.
+LAUNCH_SHAPES = [
+    (1, 40, 1, 16, 64, False, "small", "regular"),
+    (40, 130, 4, 16, 64, True, "small", "regular"),     # waves past the last query, two workgroups per head
+    (50, 150, 4, 32, 32, False, "small", "regular"),
+    (60, 190, 2, 16, 32, True, "small", "regular"),
+    (1, 65, 2, 64, 64, True, "regular", "regular"),     # four waves, a second tile of one key
+    (1, 193, 1, 16, 64, False, "split", "regular"),     # four tiles, the last of one key
+    (1, 195, 2, 32, 128, True, "split", "regular"),
+    (1, 321, 2, 64, 32, True, "split", "split"),        # six tiles
+    (1, 1000, 3, 16, 32, True, "split", "split"),
+    (2, 900, 2, 64, 64, False, "split", "split"),       # fifteen tiles: one more for the first group
+    (1, 700, 2, 32, 128, True, "split", "split"),
+    (1, 2500, 20, 16, 64, True, "split", "split"),      # up to two workgroups per CU
+    (5, 900, 8, 16, 128, False, "small", "regular"),    # wide heads
+    (9, 300, 16, 32, 128, True, "small", "regular"),    # wide heads, waves past the last query
+    (2, 257, 2, 16, 64, True, "split", "split"),        # backward: three key blocks, one key in the last
+    (1, 288, 3, 64, 32, False, "regular", "split"),     # backward: nine steps, one more for the first group
+    (1, 1100, 2, 64, 64, True, "split", "split"),       # backward: two dq tiles per wave
+    (44, 300, 2, 32, 64, True, "regular", "split"),     # two short rounds: the backward alone
+    (33, 390, 3, 16, 64, True, "small", "regular"),     # two short rounds
+    (45, 300, 3, 32, 64, True, "regular", "regular"),   # backward: eight waves on 256 keys, two key blocks, the
+    (36, 300, 3, 64, 32, True, "regular", "regular"),   # second ragged
+    (36, 300, 3, 64, 64, True, "regular", "regular"),
+    (44, 300, 2, 64, 64, False, "regular", "regular"),
+]
+
+
+@pytest.mark.parametrize("B,N,H,m,dv,causal,fwd,bwd", LAUNCH_SHAPES, ids=lambda v: str(v))
+def test_launch_shapes(B, N, H, m, dv, causal, fwd, bwd):
+    """The launch shapes of forward and backward against the oracle, on the
+    reference path (default gates) and the exact-maximum path (signed gates; 2
+    sigma keeps the scores of m = 64 in the fp32 oracle's range)."""
     for gates in (None, (0.0, 2.0)):
-        _say(f"[case] launch shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} gates={gates}")
+        _say(f"[case] launch shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} {fwd}/{bwd} gates={gates}")
         x, params, dout = make_inputs(B, N, H * dv, H, m, seed=5300 + N, gates=gates)
         scale = m ** -0.5 if gates is None else 0.5 * m ** -0.5
         out, lse, grads = run_hip(x, params, H, m, scale, causal, dout)
