@@ -145,13 +145,17 @@ constexpr bool fwd_has_split(int M, int DV) { return !(M == 64 && DV == 128); } 
 // 20.6, unmasked B1 H16 N4096 90.1 -> 92.5. From four key tiles on, six where the
 // other shape has 128 queries per workgroup anyway (mean time against not
 // split, at N64 1.04 and 1.11, N128 1.03 and 1.10, N256 0.99 and 1.04, N385 0.95 and
-// 0.99). Small below two regular workgroups per CU (m32 dv128, B1 H8 N2048 causal
-// 54.4 -> 40.9; above that, at two per CU, dv128 N4096 H16 135.6 -> 145.2).
+// 0.99). Small below two regular workgroups per CU; at dv = 128, where the
+// eight waves of a regular workgroup fill a CU, not for one unmasked round of
+// them over more than 512 keys (regular -> small, m16: 192 workgroups N1500 41.5
+// -> 45.0, N3000 74 -> 82, 256 of N4096 115 -> 123; but 256 of N257 15.5 -> 13.7, 288
+// of N3000 153 -> 131, causal 256 of N2048 51.7 -> 44.2).
 inline int attn_fwd_shape(const Dims& d) {
   const int most_unsplit = fwd_has_small(d.M, d.DV) ? 192 : 320;
   if (fwd_has_split(d.M, d.DV) && d.N > most_unsplit && few_long_chains(d, 528)) return kFwdSplit;
-  if (fwd_has_small(d.M, d.DV) && (int64_t)((d.N + 255) / 256) * d.B * d.H < 2 * 256) return kFwdSmall;
-  return kFwdRegular;
+  const int64_t wgs = (int64_t)((d.N + 255) / 256) * d.B * d.H;
+  const bool one_round = d.DV == 128 && !d.causal && wgs <= 256 && d.N > 512;
+  return fwd_has_small(d.M, d.DV) && wgs < 2 * 256 && !one_round ? kFwdSmall : kFwdRegular;
 }
 
 // Whether the split backward exists: at dv = 128 m = 16 takes 64-query steps,

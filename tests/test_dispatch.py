@@ -129,3 +129,14 @@ def test_split_shapes_stay_where_they_gain(rules):
             for c in (False, True)]
     assert all(r["fwd"] == SPLIT and r["bwd_split"] and r["soft_fwd_split"] and r["soft_bwd_split"]
                for r in rules(long))
+
+
+def test_wide_heads_keep_one_round_of_regular_workgroups(rules):
+    """dv = 128 without the causal mask: the small shape takes up to 1.12 times
+    the regular one's time where one regular round covers the problem."""
+    cases = [(B, N, H, m, 128, c) for m in (16, 32) for N in (300, 512, 640, 1000, 1500, 3000) for B in (3, 6, 12, 24)
+             for H in (8, 16) for c in (False, True)]
+    for (B, N, H, m, dv, c), r in zip(cases, rules(cases)):
+        regular = (N + 255) // 256 * B * H
+        if r["fwd"] != SPLIT:
+            assert r["fwd"] == (REGULAR if regular >= 512 or (not c and regular <= 256 and N > 512) else SMALL)

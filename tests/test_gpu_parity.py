@@ -332,7 +332,8 @@ LAUNCH_SHAPES = [
     (2, 900, 2, 64, 64, False, "split", "split"),       # fifteen tiles: one more for the first group
     (1, 700, 2, 32, 128, True, "split", "split"),
     (1, 2500, 20, 16, 64, True, "split", "split"),      # up to two workgroups per CU
-    (5, 900, 8, 16, 128, False, "small", "regular"),    # wide heads
+    (5, 900, 8, 16, 128, False, "regular", "regular"),  # wide heads, one round
+    (10, 700, 10, 16, 128, False, "small", "regular"),  # wide heads, more than one regular round
     (9, 300, 16, 32, 128, True, "small", "regular"),    # wide heads, waves past the last query
     (2, 257, 2, 16, 64, True, "split", "split"),        # backward: three key blocks, one key in the last
     (1, 288, 3, 64, 32, False, "regular", "split"),     # backward: nine steps, one more for the first group
