@@ -107,6 +107,23 @@ def test_gpu_parity_cases_run_the_shapes_they_name(rules):
         assert (("regular", "small", "split")[r["fwd"]], "split" if r["bwd_split"] else "regular") == case[6:], case
 
 
+    from test_gpu_parity import EIGHT_WAVE_BWD, VARIANT_SHAPES
+    for case, r in zip(VARIANT_SHAPES, rules([c[:6] for c in VARIANT_SHAPES])):
+        assert (("regular", "small", "split")[r["fwd"]], "split" if r["bwd_split"] else "regular") == case[8:], case
+    B, N, H = EIGHT_WAVE_BWD
+    assert not any(r["bwd_split"] for r in rules([(B, N, H, m, dv, c) for m, dv in ((32, 64), (64, 32), (64, 64))
+                                                  for c in (False, True)]))
+
+
+def test_gpu_soft_cases_run_the_shapes_they_name(rules):
+    from test_gpu_soft import BENCHMARKED_HEADS, SOFT_SHAPES
+    for case, r in zip(SOFT_SHAPES, rules([c[:6] for c in SOFT_SHAPES])):
+        assert (bool(r["soft_fwd_split"]), bool(r["soft_bwd_split"])) == case[8:], case
+    few, many = rules([(1, 4096, H, 16, 64, True) for H in BENCHMARKED_HEADS])
+    assert few["soft_fwd_split"] and few["soft_bwd_split"]
+    assert not many["soft_fwd_split"] and not many["soft_bwd_split"]
+
+
 def test_split_shapes_stay_where_they_gain(rules):
     """No split forward for the few key tiles where one group is as fast, and no
     second round of one-per-CU workgroups for short causal chains (measured up

@@ -230,14 +230,17 @@ def test_shape_matrix(m, dv, causal):
           *oracle(x, params, H, m, 0.8, causal, dout))
 
 
+EIGHT_WAVE_BWD = (45, 300, 3)  # B, N, H; tests/test_dispatch.py checks that the rules keep these from the split shape
+
+
 @pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
 @pytest.mark.parametrize("m,dv", [(32, 64), (64, 32), (64, 64)])
 def test_eight_wave_backward_key_blocks(m, dv, causal):
-    """At m = 32 and 64 (dv <= 64) a backward workgroup has eight waves and
-    owns 256 keys, and at m = 32 only four of them have dq tiles. N = 300
-    gives two key blocks, the second ragged (44 keys, so waves past N), and
-    query steps of 32 that end ragged as well."""
-    B, N, H = 2, 300, 2
+    """At m = 32 and 64 (dv <= 64), beyond the split shape's limits, a backward
+    workgroup has eight waves and owns 256 keys, and at m = 32 only four of
+    them have dq tiles. N = 300 gives two key blocks, the second ragged (44
+    keys, so waves past N), and query steps of 32 that end ragged as well."""
+    B, N, H = EIGHT_WAVE_BWD
     _say(f"[case] eight-wave backward m={m} dv={dv} causal={causal} N={N}")
     x, params, dout = make_inputs(B, N, H * dv, H, m, seed=400 + m + dv, gates=(1.0, 0.4))
     out, lse, grads = run_hip(x, params, H, m, 0.8, causal, dout)
@@ -551,6 +554,32 @@ def test_unwired_reference_variants(projection, mask_diag, m, dv, causal):
     check(f"variant {projection} mask_diag={mask_diag} m={m} dv={dv} causal={causal}", out, lse, grads, *ref)
     if causal and mask_diag:
         assert bool((out[:, 0] == 0).all()) and bool((lse[:, 0] == -3.4028234663852886e38).all())
+
+
+# (B, N, H, m, dv, causal, projection, mask_diag, forward shape, backward
+# shape); tests/test_dispatch.py checks that the launch rules give these shapes.
+VARIANT_SHAPES = [
+    (2, 190, 2, 16, 64, True, "sigmoid", True, "small", "regular"),
+    (40, 130, 4, 16, 64, False, "hardtanh01", True, "small", "regular"),   # waves past the last query
+    (50, 150, 4, 32, 32, True, "identity", False, "small", "regular"),
+    (86, 260, 3, 16, 64, True, "hardtanh01", True, "regular", "regular"),  # two query blocks per wave
+    (1, 390, 2, 16, 64, False, "sigmoid", True, "split", "split"),
+    (45, 300, 3, 32, 64, True, "sigmoid", True, "regular", "regular"),     # eight-wave backward
+]
+
+
+@pytest.mark.parametrize("B,N,H,m,dv,causal,projection,mask_diag,fwd,bwd", VARIANT_SHAPES, ids=lambda v: str(v))
+def test_variants_in_every_launch_shape(B, N, H, m, dv, causal, projection, mask_diag, fwd, bwd):
+    """The masked diagonal and the other projections (rows on the exact
+    maximum) in each launch shape against the oracle."""
+    _say(f"[case] variant shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} {projection} "
+         f"mask_diag={mask_diag} {fwd}/{bwd}")
+    x, params, dout = make_inputs(B, N, H * dv, H, m, seed=5400 + N)
+    scale = 0.7 if m == 16 else 0.4
+    out, lse, grads = _run_variant(x, params, H, m, scale, causal, dout, projection, mask_diag)
+    ref = mo.morpho_attention_ref_grads(x, *params, H, m, scale=scale, causal=causal, dout=dout, dtype=torch.float32,
+                                        projection=projection, mask_diag=mask_diag)
+    check(f"variant shapes B={B} N={N} m={m} dv={dv} {projection} mask_diag={mask_diag}", out, lse, grads, *ref)
 
 
 @pytest.mark.parametrize("causal", [False, True])

@@ -139,13 +139,46 @@ def test_soft_ragged_lengths(N):
     (290, 64, 32, True, 1), (385, 16, 64, True, -1), (257, 32, 64, False, 1),
     (1030, 16, 32, True, 1)])                                # four waves per value column
 def test_soft_forward_tiles(N, m, dv, causal, sgn):
-    """The 64-key tiles of the product-form forward (dv <= 64) at their edges,
-    and from 257 tokens on the split shape of its backward."""
+    """The 64-key tiles of the product-form forward (dv <= 64) at their edges:
+    from two tiles on the split shape (one group of waves per workgroup:
+    test_soft_launch_shapes), and from 257 tokens on that of its backward."""
     B, H = 2, 3
     _say(f"[case] soft tiles N={N} m={m} dv={dv} causal={causal} sgn={sgn}")
     x, params, dout = _inputs(B, N, H, m, dv, seed=7000 + N)
     out, zb, grads = _run(x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
     _check(f"soft tiles N={N}", out, zb, grads, x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout)
+
+
+# (B, N, H, m, dv, causal, sgn, mask_diag, split forward, split backward);
+# tests/test_dispatch.py checks that the launch rules give these shapes.
+SOFT_SHAPES = [
+    (65, 64, 4, 16, 32, True, -1, False, False, False),    # one tile
+    (44, 65, 6, 16, 64, False, 1, False, False, False),    # one key of a second tile
+    (90, 129, 3, 16, 32, True, -1, False, False, False),   # three stages
+    (50, 200, 6, 16, 32, False, 1, False, False, False),   # three stages, four tiles, the last ragged
+    (50, 200, 6, 32, 64, True, 1, False, False, False),
+    (44, 193, 6, 64, 64, False, -1, False, False, False),  # two workgroups per CU
+    (44, 130, 6, 64, 32, True, 1, True, False, False),
+    (44, 150, 6, 16, 64, True, -1, True, False, False),
+    (33, 300, 3, 16, 64, True, 1, False, False, False),    # backward: three key blocks of one group each
+    (29, 300, 3, 64, 64, False, -1, False, False, False),
+    (44, 260, 2, 32, 32, True, 1, True, False, False),
+    (1, 300, 2, 16, 64, True, 1, True, True, True),        # the split backward with the masked diagonal
+    (2, 290, 2, 64, 32, False, -1, True, True, True),
+    (1, 385, 3, 32, 64, True, -1, True, True, True),
+]
+
+
+@pytest.mark.parametrize("B,N,H,m,dv,causal,sgn,mask_diag,fwd_split,bwd_split", SOFT_SHAPES, ids=lambda v: str(v))
+def test_soft_launch_shapes(B, N, H, m, dv, causal, sgn, mask_diag, fwd_split, bwd_split):
+    """One group of waves per workgroup and two, forward and backward (dv <=
+    64), with and without the masked diagonal."""
+    _say(f"[case] soft shapes B={B} N={N} H={H} m={m} dv={dv} causal={causal} sgn={sgn} mask_diag={mask_diag} "
+         f"split={fwd_split}/{bwd_split}")
+    x, params, dout = _inputs(B, N, H, m, dv, seed=7200 + N)
+    out, zb, grads = _run(x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout, mask_diag=mask_diag)
+    _check(f"soft shapes B={B} N={N}", out, zb, grads, x, params, 0.6, H, m, m ** -0.5, causal, sgn, dout,
+           mask_diag=mask_diag)
 
 
 def test_soft_values_of_many_long_columns():
@@ -365,16 +398,22 @@ def test_exact_switch_gradients_agree():
     assert max(rels) <= 2e-3
 
 
-@pytest.mark.parametrize("sgn", [1, -1], ids=["dilation", "erosion"])
-def test_soft_product_form_at_the_benchmarked_head_shape(sgn):
+# Heads; with 17 the kernels run one group of waves per workgroup, as at the
+# benchmarked 4 x 16 heads (tests/test_dispatch.py), with two they split.
+BENCHMARKED_HEADS = (2, 17)
+
+
+@pytest.mark.parametrize("sgn,H", [(1, BENCHMARKED_HEADS[0]), (-1, BENCHMARKED_HEADS[0]),
+                                   (1, BENCHMARKED_HEADS[1])], ids=["dilation", "erosion", "dilation-H17"])
+def test_soft_product_form_at_the_benchmarked_head_shape(sgn, H):
     """The C3 head shape the soft aggregation is benchmarked on (N = 4096,
-    cube_m = 16, dv = 64, causal, tau = 0.5; two heads, default init): the
-    product form must be the path taken (flag 0), and outputs, zb and every
-    gradient including dtau meet the bars against the fp32 oracle (evaluated
-    one head at a time: it materialises [N, N, dv] per head)."""
+    cube_m = 16, dv = 64, causal, tau = 0.5; default init): the product form
+    must be the path taken (flag 0), and outputs, zb and every gradient
+    including dtau meet the bars against the fp32 oracle (evaluated one head at
+    a time: it materialises [N, N, dv] per head)."""
     from morphottention_amd import MorphoAttention
-    B, N, H, m, dv, tau, scale = 1, 4096, 2, 16, 64, 0.5, 1.0
-    _say(f"[case] soft benchmarked head shape N={N} m={m} dv={dv} sgn={sgn:+d}")
+    B, N, m, dv, tau, scale = 1, 4096, 16, 64, 0.5, 1.0
+    _say(f"[case] soft benchmarked head shape N={N} H={H} m={m} dv={dv} sgn={sgn:+d}")
     torch.manual_seed(2)
     mod = MorphoAttention(H * dv, H, m, dtype=torch.float16, device="cpu")
     params = [t.detach().cuda() for t in (mod.W_phi, mod.gate_q, mod.gate_k, mod.W_V)]
