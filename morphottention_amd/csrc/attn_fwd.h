@@ -515,9 +515,11 @@ void attn_fwd_kernel(f16* __restrict__ qa, const f16* __restrict__ ka, const f16
       if (h32 == 0) {
         const float l2 = ltot > 0.f ? R[qb] + fast_log2(ltot) : -kFltMax;  // lse - b
         lse[rowbase + q] = ltot > 0.f ? l2 + ts[qb].x : -kFltMax;
-        // the query row's affine block becomes the backward's {1, 1, -(lse - b)}:
-        // this wave was its only reader (0 for a row without keys, whose
-        // scores the backward masks)
+        // The query row's affine block becomes the backward's {1, 1, -(lse - b)}
+        // (0 for a row without keys, whose scores the backward masks). Only this
+        // workgroup reads the row: this wave, and in the split shape the same
+        // wave of the other group. Both waited for their loads before the
+        // barrier ahead of the tile loop (__syncthreads_or).
         f16 bh_, bl_;
         split_hi_lo(ltot > 0.f ? -l2 : 0.f, bh_, bl_);
         *reinterpret_cast<f16x2*>(qa + (rowbase + q) * C::CW + M + 2) = f16x2{bh_, bl_};

@@ -71,8 +71,9 @@ int make_dims(int64_t B, int64_t N, int64_t D, int64_t H, int64_t M, float scale
   // packet's 32-bit grid size): the element-wise kernels run one thread per
   // 8 (token, feature) elements (T D / 8), the backward's gate kernel 16 per
   // token, the deterministic dq reduction one per 4 (token, head, code)
-  // values; the bounds below keep each under 2^31. They sit near what fits in
-  // memory anyway (T D = 2^34 is a 32 GiB fp16 input).
+  // values; the bounds below keep each under 2^31, and the soft aggregation's
+  // column kernel caps its own grid (soft_fvals_grid). They sit near what fits
+  // in memory anyway (T D = 2^34 is a 32 GiB fp16 input).
   if (B > kMaxTokens || N > kMaxTokens)
     return fail(MORPHO_ERR_INVALID_ARGUMENT, "problem too large: B * N must be at most 2^28 tokens");
   const int64_t T = B * N;

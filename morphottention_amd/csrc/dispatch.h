@@ -20,7 +20,7 @@ struct Dims {
   int NP;                 // N rounded up to a multiple of 64: row length of the V^T layout
   int64_t T;              // B * N tokens
   int NR;                 // rows per batch row in the forward projection's row space: N rounded up to a
-                          // multiple of 8 (make_dims)
+                          // multiple of 8 (fill_sizes)
   int64_t TR;             // B * NR rows of that space
   int HM;                 // H * M projection columns
   int CW;                 // 2 * M + 8: code row width (hi/lo split codes + affine augmentation)

@@ -3,10 +3,12 @@
 // C[m][n] = sum_k A(m, k) B(k, n) over one BM x BN output tile per workgroup
 // of 8 waves (512 threads, two per SIMD) in a WM x WN arrangement, each wave
 // owning a (BM / WM) x (BN / WN) block of 16x16 accumulators
-// (v_mfma_f32_16x16x32_f16). k advances by 64 through two LDS stages that the
-// waves fill by DMA (global_load_lds_dwordx4, 1 KiB per wave instruction):
-// the stage of k-step t + 1 is issued right after the barrier that opens
-// k-step t and lands while t is computed, so no VGPRs hold prefetched data.
+// (v_mfma_f32_16x16x32_f16). k advances by 64 through STAGES LDS stages (two;
+// three for the 128 x 256 projection tile) that the waves fill by DMA
+// (global_load_lds_dwordx4, 1 KiB per wave instruction): the stage of k-step
+// t + STAGES - 1 is issued right after the barrier that opens k-step t and
+// lands while the steps before it are computed, so no VGPRs hold prefetched
+// data.
 //
 // Why 16x16x32: sustained over the whole chip, v_mfma_f32_16x16x32_f16 runs
 // at 2.24 PFLOP/s and v_mfma_f32_32x32x16_f16 at 1.82 PFLOP/s (independent

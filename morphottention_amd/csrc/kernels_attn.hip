@@ -157,7 +157,7 @@ __device__ __forceinline__ f16x8 tfrag16(const char* tile, int k0, int mn0, int 
 }
 
 // SPLIT: two groups of four waves per 128 keys, taking the query steps in turn
-// (launch_attn_bwd_t says when).
+// (attn_bwd_split says when).
 template <int M, int DV, bool SPLIT = false>
 struct BwdCfg {
   static constexpr int CW = 2 * M + 8;

@@ -71,7 +71,7 @@ hipError_t launch_transpose_weights(const Dims& d, const f16* W_phi, const f16* 
 // exactly one round of 256 tiles), 256 x 256 otherwise, and 128 x 128 when
 // the large tiles would leave most CUs idle (few tokens: B8 N1024 D512 H8 m16
 // has 64 large tiles, 320 small ones); between them 128 x 256, where half the
-// tile halves the loss of the last round (make_dims). The 128 x 128 and 128 x
+// tile halves the loss of the last round (choose_proj_tiles). The 128 x 128 and 128 x
 // 160 tiles run two to a CU with two stages each; with four stages, one to a
 // CU, they gained 1 us or lost up to 9 (B64 N128 D1024 H16 m16 31 -> 40).
 //
@@ -81,11 +81,11 @@ hipError_t launch_transpose_weights(const Dims& d, const f16* W_phi, const f16* 
 // H16 m16: 97 MB at the end of one round of tiles) and, for code that runs
 // once per tile, instruction fetch: the value part is unrolled over a wave's
 // column blocks and loses 6 us there if each block carries its own slow paths.
-// Until now 64-row slabs of the whole tile went through LDS in fp32, two of the
-// eight waves writing at a time; proj_fwd in us, before -> after: B64 N197 D768
-// H12 m64 142 -> 80, B3 N1500 D1024 H8 m32 42.7 -> 23.8, B64 N128 D1024 H16 m16
-// 40.0 -> 31.0, B64 N1024 D768 H12 m64 256 -> 246, B4 N4096 D1024 H16 m16 55.4
-// -> 56.0 (the first two mostly from the padded rows, make_dims).
+// proj_fwd in us, with 64-row slabs of the whole tile through LDS in fp32 (two of
+// the eight waves writing at a time) and this epilogue: B64 N197 D768 H12 m64 142
+// and 80, B3 N1500 D1024 H8 m32 42.7 and 23.8 (both mostly from the padded rows,
+// fill_sizes), B64 N128 D1024 H16 m16 40.0 and 31.0, B64 N1024 D768 H12 m64 256
+// and 246, B4 N4096 D1024 H16 m16 55.4 and 56.0.
 template <int BM, int BN, int STAGES>
 using ProjGemm = Gemm<BM, BN, 4, true, true, 64, STAGES>;
 

@@ -1236,22 +1236,22 @@ constexpr int soft_fast_bwd_waves() { return DV <= 64 ? 2 : 1; }
 // queries' code rows, G in bf16 hi / lo [query][column], the row references
 // A_i and token biases) arrive by LDS DMA one step ahead, into the other of
 // two stages; the code rows' affine block begins with a 1 after the codes, so
-// they also serve as [phi_hi | 1] (the ones column at code M).
+// at m = 16 they also serve as [phi_hi | 1] (the ones column at code M).
 // The S block is read in swap23 query order so that E and ds are already
 // B operands of the products that contract over the queries: dV^T += G^T E,
-// and [dk | dcb]^T += [phi_hi | 1]^T ds (one fp16 MFMA per 16 queries; the
-// ones column gives dcb). dq_i = sum_j ds_ij phi_hi_j contracts over the keys:
+// and dk^T += phi_hi^T ds (one fp16 MFMA per 32 codes and 16 queries); dcb comes
+// from the ones column at m = 16, from VALU sums of the same fp16 ds at m = 32
+// and 64. dq_i = sum_j ds_ij phi_hi_j contracts over the keys:
 // every lane stores its key's fp16 ds row (the step's 32 queries) into a
 // dS^T tile, and the step's 16 x 16 (query, code) dq tiles, split over the
 // waves, each contract over all 128 keys of the workgroup: the A operand is
 // read from the tile with transposing reads, phi_hi of the workgroup's keys
-// is the B operand (registers), and each result element is one fp32 atomic
-// per (query, code). The code-gradient products take
+// is the B operand (in registers, at m = 64 read from LDS), and each result
+// element is one fp32 atomic per (query, code). The code-gradient products take
 // ds rounded once to fp16 and the fp16 hi codes, as the softmax backward does
 // (|ds_ij| <= sum_c |dO_ic|, well inside fp16's range): relative error ~2^-11
-// per term, against the 1e-2 bar. (Three MFMAs of hi/lo pairs each had been
-// used here; the products of G, E and F keep their bf16 hi/lo pairs, whose
-// range they need.)
+// per term, against the 1e-2 bar. The products of G, E and F take bf16 hi/lo
+// pairs, whose range they need.
 // SPLIT: two groups of four waves per 128 keys, taking the query steps in turn
 // through stages and dS^T tiles of their own; the second group's sums are added
 // to the first's at the end.
