@@ -124,6 +124,16 @@ def test_gpu_soft_cases_run_the_shapes_they_name(rules):
     assert not many["soft_fwd_split"] and not many["soft_bwd_split"]
 
 
+def test_only_the_regular_forward_sees_long_rows(rules):
+    """The small and split forwards address V^T from the head's base with 32-bit
+    lane offsets, 2 dv bytes a token; their rows stay below 2^18 tokens (a
+    static_assert has the offsets of 2^18 tokens fit), the regular shape takes
+    every accepted length (a wrapped offset reads another token's values)."""
+    cases = [(1, N, 1, m, dv, c) for N in (1 << 17, (1 << 17) + 1, 1 << 18, 16_900_000, 34_000_000, 1 << 28)
+             for m in (16, 32, 64) for dv in (32, 64, 128) for c in (False, True)]
+    assert all(r["fwd"] == REGULAR or case[1] < 1 << 18 for case, r in zip(cases, rules(cases)))
+
+
 def test_split_shapes_stay_where_they_gain(rules):
     """No split forward for the few key tiles where one group is as fast, and no
     second round of one-per-CU workgroups for short causal chains (measured up
