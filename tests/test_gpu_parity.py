@@ -310,10 +310,10 @@ def test_short_ragged_rows_cost_no_more_than_whole_ones(B, N, H, m, dv):
         for _ in range(20):
             torch.ops.morphottention.forward(x, *params, H, m, 1.0, False)
         torch.cuda.synchronize()
-        t = sorted(ms for _, ms in capi.timing_read())
+        t = [ms for _, ms in capi.timing_read()]
         capi.timing_enable(False)
         capi.timing_only(None)
-        return 1e3 * t[len(t) // 2]
+        return 1e3 * min(t)  # a dispatch after an idle moment can show 4 us more
 
     ragged, whole = proj_us(N), proj_us((N + 7) // 8 * 8)
     _say(f"[case] short rows B={B} N={N} H={H} m={m} dv={dv}: proj_fwd {ragged:.1f} us, whole groups {whole:.1f} us")
